@@ -30,10 +30,11 @@
 //                       h0*y0 + h1*y1 + bias (one slice) or adds h0*y0 +
 //                       h1*y1 to y with fp32 atomics (several slices; the
 //                       latent kernel has set y = bias + residual).
-// GEMM path (M > 64, or operands too large for the decode path's LDS):
-//   gemm_scale_kernel (bf16 g*x, when x cannot be read as it is) /
+// GEMM path (M > 64, or operands too large for the decode path's LDS), bf16
+// activations: gemm_scale_kernel (bf16 g*x, when x cannot be read as it is) /
 //   gemm_latent_kernel (or its stream-K form) / gemm_expand_kernel (or its
-//   128 x 256 tile form), tiled on v_mfma_f32_32x32x16_bf16.
+//   128 x 256 tile form), tiled on v_mfma_f32_32x32x16_bf16.  fp32
+//   activations: the kernels of split_gemm.h.
 //
 // Splitting fp32 activations into bf16 hi + lo keeps the product error near
 // 2^-17 relative: +-1 is exact in bf16 and the MFMA accumulates in fp32.
@@ -1943,16 +1944,15 @@ __global__ __launch_bounds__(W * kWave) void chain_mfma_kernel(ChainParams cp) {
 }
 
 // ---------------------------------------------------------------------------
-// GEMM path (M > 16, and shapes the decode path cannot stage in LDS): a
-// tiled sign-GEMM on v_mfma_f32_32x32x16_bf16, three launches per call.
+// GEMM path on bf16 activations (M > 64, and shapes the decode path cannot
+// stage in LDS; fp32 activations: split_gemm.h): a tiled sign-GEMM on
+// v_mfma_f32_32x32x16_bf16, three launches per call.
 //   prologue  A_s[m, k] = g_s[k] * x[m, k] per branch s, as bf16, k padded
 //             with zeros to a multiple of 64
 //   stage 1   T_s[m, r] = l_s[r] * sum_k sV_s[r, k] * A_s[m, k], as bf16
 //   stage 2   y[m, n] = bias[n] + sum_b h_b[n] * sum_r sU_b[n, r] * T_b[m, r]
-// With SPLIT (fp32 activations) A and T are stored as two bf16 planes, hi
-// and lo = bf16(v - hi), and both planes go through the MFMA, so products
-// keep ~2^-17 relative error.  Without SPLIT (bf16 activations) one plane:
-// the precision of the reference's bf16 forward (littlebit.py:116-121).
+// One bf16 plane each: the precision of the reference's bf16 forward
+// (littlebit.py:116-121).
 // Stages 1 and 2: block tile 128 (m) x 128 (columns: latent rows in stage
 // 1, outputs in stage 2), 4 waves of 64 x 64 (2 x 2 MFMA tiles), k-steps of
 // 64.  A tiles go from global memory straight to LDS through a 4-stage ring
@@ -2004,21 +2004,13 @@ struct GemmParams {
   const void* x1;
   const float* nw;
   float eps;
-  uint16_t* a;        // A planes (hi, then lo with SPLIT)
-  uint16_t* t;        // T planes
-  int64_t a_plane;    // elements per A plane
-  int64_t t_plane;    // elements per T plane
+  uint16_t* a;        // A
+  uint16_t* t;        // T
 };
-
-// hi = bf16(v), lo = bf16(v - hi), round to nearest even
-__device__ __forceinline__ void split1(float v, uint16_t& hi, uint16_t& lo) {
-  hi = f32_to_bf16(v);
-  lo = f32_to_bf16(v - bf16_to_f32(hi));
-}
 
 // Prologue.  grid = (M, segments), 256 threads; thread handles 8-k chunks.
 // The input mode (RMSNorm, SiLU * up) is applied here, as in load_input8.
-template <typename XT, bool SPLIT>
+template <typename XT>
 __global__ __launch_bounds__(kGThreads) void gemm_scale_kernel(GemmParams p) {
   const int m = int(blockIdx.x);
   const GemmSeg& S = p.seg[__builtin_amdgcn_readfirstlane(int(blockIdx.y))];
@@ -2066,17 +2058,10 @@ __global__ __launch_bounds__(kGThreads) void gemm_scale_kernel(GemmParams p) {
         v[i] = e;
       }
     }
-    if constexpr (SPLIT) {
-      u32x4 h, l;
-      split8(v, h, l);
-      *reinterpret_cast<u32x4*>(hi + k) = h;
-      *reinterpret_cast<u32x4*>(hi + p.a_plane + k) = l;
-    } else {
-      u32x4 h;
+    u32x4 h;
 #pragma unroll
-      for (int d = 0; d < 4; ++d) h[d] = uint32_t(f32_to_bf16(v[2 * d])) | (uint32_t(f32_to_bf16(v[2 * d + 1])) << 16);
-      *reinterpret_cast<u32x4*>(hi + k) = h;
-    }
+    for (int d = 0; d < 4; ++d) h[d] = uint32_t(f32_to_bf16(v[2 * d])) | (uint32_t(f32_to_bf16(v[2 * d + 1])) << 16);
+    *reinterpret_cast<u32x4*>(hi + k) = h;
   }
 }
 
@@ -2151,8 +2136,8 @@ __device__ __forceinline__ int gemm_col(int wn, int j) {
 __device__ __forceinline__ int gemm_wm(int wave) { return kGWM == 1 ? 0 : wave >> 1; }
 __device__ __forceinline__ int gemm_wn(int wave) { return kGWM == 1 ? wave : wave & 1; }
 
-template <bool SPLIT, bool GB = false, int BN = 128>
-__device__ __forceinline__ void gemm_mainloop(const uint16_t* __restrict__ A, int64_t plane, int64_t lda, int M,
+template <bool GB = false, int BN = 128>
+__device__ __forceinline__ void gemm_mainloop(const uint16_t* __restrict__ A, int64_t lda, int M,
                                               int m0, const uint32_t* __restrict__ W, int ldw, int ncols, int c0,
                                               int nks, f32x16 (&acc)[kGMI][gemm_nj<BN>()], int tid,
                                               const float* __restrict__ g = nullptr, int kbase = 0,
@@ -2163,14 +2148,13 @@ __device__ __forceinline__ void gemm_mainloop(const uint16_t* __restrict__ A, in
   constexpr int NJ = gemm_nj<BN>();
   typedef __attribute__((address_space(3))) void* lds_ptr_t;
   typedef __attribute__((address_space(1))) void* glb_ptr_t;
-  constexpr int NT = SPLIT ? 2 : 1;
   constexpr int NW = BN / 128;              // sign words per thread and step
-  constexpr int TILE = kGB * kGK;           // elements per plane per stage
-  constexpr int LOADS_PER_FILL = 4 * NT + NW + (GB ? 1 : 0);  // global_load_lds, sign words, g; per wave
-  __shared__ __attribute__((aligned(16))) uint16_t st0[NT * TILE];
-  __shared__ __attribute__((aligned(16))) uint16_t st1[NT * TILE];
-  __shared__ __attribute__((aligned(16))) uint16_t st2[NT * TILE];
-  __shared__ __attribute__((aligned(16))) uint16_t st3[NT * TILE];
+  constexpr int TILE = kGB * kGK;           // elements per stage
+  constexpr int LOADS_PER_FILL = 4 + NW + (GB ? 1 : 0);  // global_load_lds, sign words, g; per wave
+  __shared__ __attribute__((aligned(16))) uint16_t st0[TILE];
+  __shared__ __attribute__((aligned(16))) uint16_t st1[TILE];
+  __shared__ __attribute__((aligned(16))) uint16_t st2[TILE];
+  __shared__ __attribute__((aligned(16))) uint16_t st3[TILE];
   __shared__ __attribute__((aligned(16))) uint32_t sw[2][2 * BN];
   __shared__ __attribute__((aligned(16))) uint16_t gb[2][kGK];
   const int lane = tid & 63;
@@ -2243,9 +2227,6 @@ __device__ __forceinline__ void gemm_mainloop(const uint16_t* __restrict__ A, in
     for (int j = 0; j < 4; ++j) {
       uint16_t* dst = st + (wave * 4 + j) * 512;
       __builtin_amdgcn_global_load_lds((glb_ptr_t)(src[j] + int64_t(kbase + ks) * kGK), (lds_ptr_t)dst, 16, 0, 0);
-      if constexpr (SPLIT)
-        __builtin_amdgcn_global_load_lds((glb_ptr_t)(src[j] + plane + int64_t(kbase + ks) * kGK), (lds_ptr_t)(dst + TILE),
-                                         16, 0, 0);
     }
   };
   uint32_t kmask = 0x80008000u, kone = 0x3F803F80u;
@@ -2279,12 +2260,6 @@ __device__ __forceinline__ void gemm_mainloop(const uint16_t* __restrict__ A, in
         const bf16x8 ah = *reinterpret_cast<const bf16x8*>(a + off);
 #pragma unroll
         for (int j = 0; j < NJ; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah, b[j], acc[i][j], 0, 0, 0);
-        if constexpr (SPLIT) {
-          const bf16x8 al = *reinterpret_cast<const bf16x8*>(a + TILE + off);
-#pragma unroll
-          for (int j = 0; j < NJ; ++j)
-            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(al, b[j], acc[i][j], 0, 0, 0);
-        }
       }
     }
   };
@@ -2341,7 +2316,6 @@ __device__ __forceinline__ void gemm_mainloop(const uint16_t* __restrict__ A, in
 // Stage 1 epilogue: T rows of the tile (m0, c0) of segment G, l-scaled.
 constexpr int kGNJ = gemm_nj<kGB>();  // column tiles per wave of a 128-column block
 
-template <bool SPLIT>
 __device__ __forceinline__ void latent_store(const GemmParams& p, const GemmSeg& G, int m0, int c0,
                                              const f32x16 (&acc)[kGMI][kGNJ], int tid) {
   const int lane = tid & 63, wave = tid >> 6;
@@ -2360,14 +2334,7 @@ __device__ __forceinline__ void latent_store(const GemmParams& p, const GemmSeg&
         if (m < p.M) {
           const int64_t o = int64_t(m) * G.RP + r;
           const float v = lv * acc[i][j][q];
-          if constexpr (SPLIT) {
-            uint16_t h, l;
-            split1(v, h, l);
-            T[o] = h;
-            T[p.t_plane + o] = l;
-          } else {
-            T[o] = f32_to_bf16(v);
-          }
+          T[o] = f32_to_bf16(v);
         }
       }
   }
@@ -2383,7 +2350,7 @@ __device__ __forceinline__ int latent_segment(const GemmParams& p, int nt) {
 // Stage 1.  grid = (m-tiles, column tiles of all segments), 256 threads.
 // GB: A is the bf16 input itself (every segment's abase 0, rows of Kp = K)
 // and g goes into the B operand.
-template <bool SPLIT, bool GB>
+template <bool GB>
 __global__ __launch_bounds__(kGThreads) void gemm_latent_kernel(GemmParams p) {
   const int tid = int(threadIdx.x);
   const int nt = int(blockIdx.y);
@@ -2395,8 +2362,8 @@ __global__ __launch_bounds__(kGThreads) void gemm_latent_kernel(GemmParams p) {
   for (int i = 0; i < kGMI; ++i)
 #pragma unroll
     for (int j = 0; j < kGNJ; ++j) acc[i][j] = f32x16{};
-  gemm_mainloop<SPLIT, GB>(p.a + G.abase, p.a_plane, p.Kp, p.M, m0, G.V, p.KW, G.R, c0, p.Kp / kGK, acc, tid, G.g);
-  latent_store<SPLIT>(p, G, m0, c0, acc, tid);
+  gemm_mainloop<GB>(p.a + G.abase, p.Kp, p.M, m0, G.V, p.KW, G.R, c0, p.Kp / kGK, acc, tid, G.g);
+  latent_store(p, G, m0, c0, acc, tid);
 }
 
 // Stage 1, stream-K form: when the tiles do not fill the CUs' block slots
@@ -2435,7 +2402,7 @@ __device__ __forceinline__ int sk_block(int64_t i, const SkParams& q) { return i
 
 // Two blocks per CU (the sk_blocks plan assumes them): held to 256 registers
 // per lane (unbounded, the partial-tile code took 256 VGPRs + 64 AGPRs).
-template <bool SPLIT, bool GB>
+template <bool GB>
 __global__ __launch_bounds__(kGThreads, 2) void gemm_latent_sk_kernel(GemmParams p, SkParams q) {
   const int tid = int(threadIdx.x);
   const int grp = int(blockIdx.x) % q.G;
@@ -2456,7 +2423,7 @@ __global__ __launch_bounds__(kGThreads, 2) void gemm_latent_sk_kernel(GemmParams
     for (int i = 0; i < kGMI; ++i)
 #pragma unroll
       for (int j = 0; j < kGNJ; ++j) acc[i][j] = f32x16{};
-    gemm_mainloop<SPLIT, GB>(p.a + G.abase, p.a_plane, p.Kp, p.M, m0, G.V, p.KW, G.R, c0, n, acc, tid, G.g, k0);
+    gemm_mainloop<GB>(p.a + G.abase, p.Kp, p.M, m0, G.V, p.KW, G.R, c0, n, acc, tid, G.g, k0);
     bool store = true;
     if (n < q.nks) {
       const int64_t ts = int64_t(t) * q.nks;
@@ -2502,7 +2469,7 @@ __global__ __launch_bounds__(kGThreads, 2) void gemm_latent_sk_kernel(GemmParams
         if (tid == 0) __hip_atomic_store(q.cnt + gb0 + bf, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       }
     }
-    if (store) latent_store<SPLIT>(p, G, m0, c0, acc, tid);
+    if (store) latent_store(p, G, m0, c0, acc, tid);
     it += n;
   }
 }
@@ -2510,7 +2477,7 @@ __global__ __launch_bounds__(kGThreads, 2) void gemm_latent_sk_kernel(GemmParams
 // Stage 2.  grid = (m-tiles, column tiles of all projections), 256 threads.
 // Held to 256 registers per lane (two waves per SIMD; unbounded, the two
 // accumulator sets took 244 VGPRs + 64 AGPRs, one wave per SIMD).
-template <typename YT, bool SPLIT>
+template <typename YT>
 __global__ __launch_bounds__(kGThreads, 2) void gemm_expand_kernel(GemmParams p) {
   const int tid = int(threadIdx.x);
   const int nt = int(blockIdx.y);
@@ -2527,10 +2494,10 @@ __global__ __launch_bounds__(kGThreads, 2) void gemm_expand_kernel(GemmParams p)
 #pragma unroll
     for (int j = 0; j < kGNJ; ++j) acc0[i][j] = acc1[i][j] = f32x16{};
   // T rows are zero from R to RP >= 64 * ceil(RW / 2), so whole 64-k steps are safe
-  gemm_mainloop<SPLIT>(p.t + P.tbase[0], p.t_plane, P.RP[0], p.M, m0, P.U[0], P.RW[0], P.N, c0, (P.RW[0] + 1) / 2,
+  gemm_mainloop<>(p.t + P.tbase[0], P.RP[0], p.M, m0, P.U[0], P.RW[0], P.N, c0, (P.RW[0] + 1) / 2,
                        acc0, tid);
   if (P.nb > 1)
-    gemm_mainloop<SPLIT>(p.t + P.tbase[1], p.t_plane, P.RP[1], p.M, m0, P.U[1], P.RW[1], P.N, c0,
+    gemm_mainloop<>(p.t + P.tbase[1], P.RP[1], p.M, m0, P.U[1], P.RW[1], P.N, c0,
                          (P.RW[1] + 1) / 2, acc1, tid);
 
   const int lane = tid & 63, wave = tid >> 6;
@@ -2588,7 +2555,7 @@ __global__ __launch_bounds__(kGThreads, 2) void gemm_expand_wide_kernel(GemmPara
 #pragma unroll
     for (int j = 0; j < NJ; ++j) acc[i][j] = f32x16{};
   // T rows are zero from R to RP >= 64 * ceil(RW / 2), so whole 64-k steps are safe
-  gemm_mainloop<false, false, BN>(p.t + P.tbase[0], p.t_plane, P.RP[0], p.M, m0, P.U[0], P.RW[0], P.N, c0,
+  gemm_mainloop<false, BN>(p.t + P.tbase[0], P.RP[0], p.M, m0, P.U[0], P.RW[0], P.N, c0,
                                   (P.RW[0] + 1) / 2, acc, tid, nullptr, 0, nullptr);
   float f[NJ];  // the factor y takes of acc, per subtile column
 #pragma unroll
@@ -2605,7 +2572,7 @@ __global__ __launch_bounds__(kGThreads, 2) void gemm_expand_wide_kernel(GemmPara
     }
   }
   if (P.nb > 1)
-    gemm_mainloop<false, false, BN>(p.t + P.tbase[1], p.t_plane, P.RP[1], p.M, m0, P.U[1], P.RW[1], P.N, c0,
+    gemm_mainloop<false, BN>(p.t + P.tbase[1], P.RP[1], p.M, m0, P.U[1], P.RW[1], P.N, c0,
                                     (P.RW[1] + 1) / 2, acc, tid, nullptr, 0, P.h[1], P.h[0]);
 
   YT* __restrict__ y = static_cast<YT*>(P.y);
@@ -2627,6 +2594,14 @@ __global__ __launch_bounds__(kGThreads, 2) void gemm_expand_wide_kernel(GemmPara
       }
   }
 }
+
+// hi = bf16(v), lo = bf16(v - hi), round to nearest even
+__device__ __forceinline__ void split1(float v, uint16_t& hi, uint16_t& lo) {
+  hi = f32_to_bf16(v);
+  lo = f32_to_bf16(v - bf16_to_f32(hi));
+}
+
+#include "split_gemm.h"
 
 // ---------------------------------------------------------------------------
 // Sign pack / unpack (bit-exact with the reference packer)
@@ -3609,6 +3584,7 @@ struct Plan {
   bool seq;      // chunk > 0: one launch pair per chunk, one chunk after another
   bool reverse;  // seq: the chunks run last to first (an output overlapping the input)
   size_t lds1, lds2;
+  bool split;    // seq: the rows run on the split GEMM path where the workspace holds it
   size_t ws_total;  // workspace the fastest form of the call uses
   size_t ws_min;    // workspace it needs (GEMM path: without the stream-K partial tiles)
 };
@@ -3623,7 +3599,7 @@ size_t compact_rows(int mt, int64_t nch) {
 
 
 // Elements per plane of the GEMM path's A (per segment [M][Kp]) and T (per
-// segment [M][RP]); planes are bf16, two of each with SPLIT.
+// segment [M][RP]); planes are bf16, two of each (hi, lo) for fp32 activations.
 void gemm_planes(const ProjDesc* pd, int np, int64_t M, int64_t K, int64_t& a_plane, int64_t& t_plane) {
   a_plane = t_plane = 0;
   const int64_t Kp = ceil_div(K, kGK) * kGK;
@@ -3634,11 +3610,60 @@ void gemm_planes(const ProjDesc* pd, int np, int64_t M, int64_t K, int64_t& a_pl
     }
 }
 
-size_t gemm_ws_bytes(const ProjDesc* pd, int np, int64_t M, int64_t K, bool split) {
+// Room for two planes of each (a query does not know the activations' type).
+size_t gemm_ws_bytes(const ProjDesc* pd, int np, int64_t M, int64_t K) {
   int64_t ap, tp;
   gemm_planes(pd, np, M, K, ap, tp);
-  const size_t planes = split ? 2 : 1;
-  return align256(size_t(ap) * planes * sizeof(uint16_t)) + align256(size_t(tp) * planes * sizeof(uint16_t));
+  return align256(size_t(ap) * 2 * sizeof(uint16_t)) + align256(size_t(tp) * 2 * sizeof(uint16_t));
+}
+
+// Launch shape of the split GEMM path (split_gemm.h), from a sweep of every
+// (rows, columns, parts) over single and grouped Llama-2 / Llama-3 calls, one
+// and two branches, M = 33 .. 2048; the choices are within about 5 % of the
+// best shape of each stage.  Tiles are counted as 32 x 128.
+//   Stage 1: 32 x 128 tiles, the k range in parts while there are fewer than
+//   about 512 blocks (two per CU): M = 300, one 4096 -> 4096 projection of
+//   ranks 205 + 1843, 170 tiles, 24.5 us whole and 22.2 us in 3 parts; M =
+//   2048, gate and up, 3072 tiles, 178.6 us against 167.3 us in 64-row tiles.
+//   Stage 2: 32 x 128 tiles while they are few (M = 512, 4096 columns: 512
+//   tiles 22.2 us, 64 x 128 27.1 us, 64 x 256 43.8 us) or the ranks are short
+//   (each tile then mostly stores y), 64 x 256 where those give 600 blocks (M
+//   = 1024, gate and up: 217.6 us against 227.4 us as 64 x 128 and 251.5 us
+//   as 32 x 128), else 64 x 128.
+struct SgPlan {
+  int mi1, parts;  // stage 1: 32 mi1 rows x 128 columns, parts of the k range
+  int mi2, nj2;    // stage 2: 32 mi2 rows x 128 nj2 columns
+  size_t part_bytes;
+};
+SgPlan sg_plan(const ProjDesc* pd, int np, int64_t M, int64_t K) {
+  int64_t c1 = 0, cols = 0, c2 = 0, c2w = 0, steps = 0;
+  for (int q = 0; q < np; ++q) {
+    int64_t st = 0;
+    for (int b = 0; b < pd[q].nb; ++b) {
+      const int64_t R = pd[q].br[b].rank;
+      c1 += ceil_div(R, 128);
+      st += ceil_div(R, 32);
+    }
+    c2 += ceil_div(pd[q].N, 128);
+    c2w += ceil_div(pd[q].N, 256);
+    steps = std::max(steps, st);
+  }
+  cols = 128 * c1;
+  SgPlan s{};
+  const int64_t tiles1 = std::max<int64_t>(1, ceil_div(M, 32)) * c1;  // M = 0: a query
+  s.mi1 = tiles1 < 1500 ? 1 : 2;
+  s.parts = 1;
+  if (s.mi1 == 1) {
+    const int64_t groups = ceil_div(K, 128);  // at least two groups of steps per part
+    s.parts = int(std::max<int64_t>(1, std::min<int64_t>({(512 + tiles1 / 2) / tiles1, 8, groups / 2})));
+  }
+  s.part_bytes = s.parts > 1 ? size_t(s.parts) * size_t(M) * size_t(cols) * sizeof(float) : 0;
+  s.mi2 = s.nj2 = 1;
+  if (ceil_div(M, 32) * c2 > 1100 && steps > 16) {
+    s.mi2 = 2;
+    s.nj2 = ceil_div(M, 64) * c2w >= 600 ? 2 : 1;
+  }
+  return s;
 }
 
 // Static LDS of expand_mfma_kernel (the `red` array).
@@ -3843,10 +3868,10 @@ Plan plan_one(const ProjDesc* pd, int np, int64_t M, int64_t K, bool allow_ks, b
     if (det && pl.nkc > 1)
       pl.ws_total = pl.ws_min = kGemmOffset + align256(det_part_floats(pd, np, M, pl.nkc) * sizeof(float));
   } else {
-    pl.ws_min = kGemmOffset + gemm_ws_bytes(pd, np, M, K, true);
+    pl.ws_min = kGemmOffset + gemm_ws_bytes(pd, np, M, K);
     const int64_t tiles = ceil_div(M, kGB) * latent_col_tiles(pd, np), nks = ceil_div(K, kGK);
-    const int64_t P = std::max(sk_blocks(tiles, nks, 2 * kNumCUs), sk_blocks(tiles, nks, kNumCUs));
-    pl.ws_total = pl.ws_min + size_t(2 * P) * kSkSlotBytes;
+    const int64_t P = sk_blocks(tiles, nks, 2 * kNumCUs);
+    pl.ws_total = pl.ws_min + std::max(size_t(2 * P) * kSkSlotBytes, sg_plan(pd, np, M, K).part_bytes);
   }
   return pl;
 }
@@ -3857,6 +3882,8 @@ Plan plan_one(const ProjDesc* pd, int np, int64_t M, int64_t K, bool allow_ks, b
 // blocks for the latent stage of a Llama-2 o projection at M = 33).  Rows of
 // a call are independent, so the chunks compute what one call would.
 constexpr int64_t kMaxChunkedM = 64;
+
+size_t sg_ws_bytes(const ProjDesc* pd, int np, int64_t M, int64_t K);
 
 // Whether M rows of the projections' latent vectors and their sums of
 // squares fit one latent half.
@@ -3871,7 +3898,10 @@ bool t_fits(const ProjDesc* pd, int np, int64_t M) {
 // measured 16 % faster than 16-row chunks at 17-40 rows of the Llama-2 target
 // calls), else 16 (one launch pair per chunk: fewer pairs).  Side by side,
 // 9-16 rows also go as 8-row chunks rather than one 16-row pass (measured 6-11
-// % faster at 9, 12 and 16 rows over the draft and target calls).
+// % faster at 9, 12 and 16 rows over the draft and target calls).  More than
+// 32 rows that would run as 16-row chunks one after another take the split
+// GEMM path instead (64 rows of the target's q/k/v 178 -> 47 us, gate/up 310
+// -> 61 us), as long as the workspace holds its planes.
 Plan make_plan(const ProjDesc* pd, int np, int64_t M, int64_t K, bool allow_ks, bool det) {
   const Plan pl = plan_one(pd, np, M, K, allow_ks, det);
   const bool side_by_side = !det && t_fits(pd, np, M);
@@ -3882,6 +3912,8 @@ Plan make_plan(const ProjDesc* pd, int np, int64_t M, int64_t K, bool allow_ks, 
       if (pc.mfma) {
         pc.chunk = int(c);
         pc.seq = !side_by_side;
+        pc.split = pc.seq && M > 2 * kMaxMfmaM;
+        if (pc.split) pc.ws_total = std::max(pc.ws_total, sg_ws_bytes(pd, np, M, K));
         return pc;
       }
     }
@@ -4061,9 +4093,112 @@ int forward_mfma(const ProjDesc* pd, int np, const Plan& pl, int64_t M, int64_t 
   return check_launch("expand_mfma_kernel");
 }
 
+template <typename YT>
+void launch_sg_expand(const SgParams& p, const SgPlan& sp, dim3 grid, hipStream_t s) {
+  if (sp.nj2 == 2) hipLaunchKernelGGL((sg_expand_kernel<YT, 2, 2>), grid, dim3(kBlock), 0, s, p);
+  else if (sp.mi2 == 2) hipLaunchKernelGGL((sg_expand_kernel<YT, 2, 1>), grid, dim3(kBlock), 0, s, p);
+  else hipLaunchKernelGGL((sg_expand_kernel<YT, 1, 1>), grid, dim3(kBlock), 0, s, p);
+}
+
+// Workspace of a split-GEMM call: A and T, then stage 1's parts.
+size_t sg_ws_bytes(const ProjDesc* pd, int np, int64_t M, int64_t K) {
+  return kGemmOffset + gemm_ws_bytes(pd, np, M, K) + sg_plan(pd, np, M, K).part_bytes;
+}
+
+// A call on the split GEMM path (split_gemm.h).  x is read by the first
+// kernel only, so an output may share its memory.  A workspace without room
+// for stage 1's parts runs whole tiles.
+int forward_split(const ProjDesc* pd, int np, int64_t M, int64_t K, const void* x, int x_dtype, const InputDesc& in,
+                  int y_dtype, void* workspace, size_t workspace_bytes, hipStream_t s) {
+  SgPlan sp = sg_plan(pd, np, M, K);
+  const size_t planes = gemm_ws_bytes(pd, np, M, K);
+  if (sp.parts > 1 && workspace_bytes < kGemmOffset + planes + sp.part_bytes) sp.parts = 1;
+  SgParams p;
+  memset(&p, 0, sizeof(p));
+  p.nproj = np;
+  p.M = int(M);
+  p.K = int(K);
+  p.KW = int(ceil_div(K, 32));
+  p.lda = 64 * p.KW;
+  p.x = x;
+  p.x1 = in.x1;
+  p.nw = in.nw;
+  p.eps = in.eps;
+  p.xmode = in.kind;
+  bool xvec = (K % 8) == 0 && aligned16(x) && (!in.x1 || aligned16(in.x1)) && (!in.nw || aligned16(in.nw));
+  int64_t abase = 0, nt1 = 0, nt2 = 0;
+  int si = 0, tcol = 0;
+  for (int q = 0; q < np; ++q) {
+    SgProj& P = p.proj[q];
+    P.nb = pd[q].nb;
+    P.N = int(pd[q].N);
+    P.bias = pd[q].bias;
+    P.res = pd[q].res;
+    P.y = pd[q].y;
+    P.tcol = tcol;
+    P.nt0 = int(nt2);
+    nt2 += ceil_div(pd[q].N, 128 * sp.nj2);
+    for (int b = 0; b < pd[q].nb; ++b, ++si) {
+      const lbk_branch& B = pd[q].br[b];
+      SgSeg& S = p.seg[si];
+      S.V = reinterpret_cast<const uint32_t*>(B.v_sign);
+      S.Vt = reinterpret_cast<const uint32_t*>(B.v_sign_tiled);
+      S.g = B.v2;
+      S.l = B.mid;
+      S.R = int(B.rank);
+      P.U[b] = reinterpret_cast<const uint32_t*>(B.u_sign);
+      P.h[b] = B.u1;
+      P.RW[b] = int(ceil_div(B.rank, 32));
+      P.ng[b] = int(ceil_div(B.rank, 128));
+      S.RP = 128 * P.ng[b];
+      S.tcol = tcol;
+      S.nt0 = int(nt1);
+      S.abase = abase;
+      nt1 += P.ng[b];
+      tcol += S.RP;
+      abase += M * p.lda;
+      xvec = xvec && (reinterpret_cast<uintptr_t>(B.v2) % 16) == 0;
+    }
+  }
+  p.nseg = si;
+  p.ldt = 2 * tcol;
+  p.xvec = xvec ? 1 : 0;
+  char* ws = static_cast<char*>(workspace) + kGemmOffset;
+  p.a = reinterpret_cast<uint16_t*>(ws);
+  p.t = reinterpret_cast<uint16_t*>(ws + align256(size_t(abase) * sizeof(uint16_t)));
+  p.part = reinterpret_cast<float*>(ws + planes);
+  const int64_t blocks1 = ceil_div(M, 32 * sp.mi1) * nt1 * sp.parts, blocks2 = ceil_div(M, 32 * sp.mi2) * nt2;
+  if (nt1 > 65535 || ceil_div(nt2, 2) > 65535 || blocks1 > INT_MAX || blocks2 > INT_MAX)
+    return set_error(LBK_ERR_ARG, "too many column tiles for the GEMM path");
+
+  const dim3 g0(unsigned(M), unsigned(ceil_div(p.KW, 64)));
+  if (x_dtype == LBK_F32) hipLaunchKernelGGL(sg_scale_kernel<float>, g0, dim3(kBlock), 0, s, p);
+  else hipLaunchKernelGGL(sg_scale_kernel<uint16_t>, g0, dim3(kBlock), 0, s, p);
+  int rc = check_launch("sg_scale_kernel");
+  if (rc != LBK_OK) return rc;
+  p.parts = sp.parts;
+  p.NT = int(nt1);
+  const dim3 g1{unsigned(blocks1), 1u, 1u}, g2{unsigned(blocks2), 1u, 1u};
+  if (sp.mi1 == 1) hipLaunchKernelGGL(sg_latent_kernel<1>, g1, dim3(kBlock), 0, s, p);
+  else hipLaunchKernelGGL(sg_latent_kernel<2>, g1, dim3(kBlock), 0, s, p);
+  rc = check_launch("sg_latent_kernel");
+  if (rc != LBK_OK) return rc;
+  if (sp.parts > 1) {
+    const dim3 gr(unsigned(ceil_div(M * tcol, 4 * kBlock)));
+    hipLaunchKernelGGL(sg_reduce_t_kernel, gr, dim3(kBlock), 0, s, p);
+    rc = check_launch("sg_reduce_t_kernel");
+    if (rc != LBK_OK) return rc;
+  }
+  p.parts = 1;
+  p.NT = int(nt2);
+  if (y_dtype == LBK_F32) launch_sg_expand<float>(p, sp, g2, s);
+  else launch_sg_expand<uint16_t>(p, sp, g2, s);
+  return check_launch("sg_expand_kernel");
+}
+
 int forward_gemm(const ProjDesc* pd, int np, int64_t M, int64_t K, const void* x, int x_dtype, const InputDesc& in,
                  int y_dtype, void* workspace, size_t workspace_bytes, hipStream_t s) {
-  const bool split = x_dtype == LBK_F32;
+  if (x_dtype == LBK_F32) return forward_split(pd, np, M, K, x, x_dtype, in, y_dtype, workspace, workspace_bytes, s);
   GemmParams p;
   memset(&p, 0, sizeof(p));
   p.nproj = np;
@@ -4072,10 +4207,11 @@ int forward_gemm(const ProjDesc* pd, int np, int64_t M, int64_t K, const void* x
   p.KW = int(ceil_div(K, 32));
   p.Kp = int(ceil_div(K, kGK) * kGK);
   p.x = x;
-  gemm_planes(pd, np, M, K, p.a_plane, p.t_plane);
+  int64_t a_plane, t_plane;
+  gemm_planes(pd, np, M, K, a_plane, t_plane);
   char* ws = static_cast<char*>(workspace) + kGemmOffset;
   p.a = reinterpret_cast<uint16_t*>(ws);
-  p.t = reinterpret_cast<uint16_t*>(ws + align256(size_t(p.a_plane) * (split ? 2 : 1) * sizeof(uint16_t)));
+  p.t = reinterpret_cast<uint16_t*>(ws + align256(size_t(a_plane) * sizeof(uint16_t)));
   p.xmode = in.kind;
   p.x1 = in.x1;
   p.nw = in.nw;
@@ -4123,15 +4259,14 @@ int forward_gemm(const ProjDesc* pd, int np, int64_t M, int64_t K, const void* x
   const dim3 g1{unsigned(mtiles), unsigned(nt1), 1u}, g2{unsigned(mtiles), unsigned(nt2), 1u};
   // bf16 rows of whole k-steps, taken as they are: g goes into stage 1's B
   // operand and no scaled copy of x is made
-  const bool direct = !split && in.kind == LBK_INPUT_PLAIN && K % kGK == 0 && aligned16(x);
+  const bool direct = in.kind == LBK_INPUT_PLAIN && K % kGK == 0 && aligned16(x);
   // Stream-K stage 1 when whole tiles would leave the block slots unevenly
   // used (estimated in k-steps of one block: rounds of tiles vs an even
   // share plus about two steps for the partial tiles), and the workspace
   // holds the partial tiles.
   const int64_t nks = p.Kp / kGK, tiles = mtiles * nt1;
-  const int slots = (split ? 1 : 2) * kNumCUs;  // blocks resident at once (LDS of the stage ring)
-  const size_t part_off = kGemmOffset + gemm_ws_bytes(pd, np, M, K, true);
-  const int64_t P = sk_blocks(tiles, nks, slots);
+  const size_t part_off = kGemmOffset + gemm_ws_bytes(pd, np, M, K);
+  const int64_t P = sk_blocks(tiles, nks, 2 * kNumCUs);  // blocks resident at once (LDS of the stage ring)
   const bool sk = P > 0 && workspace_bytes >= part_off + size_t(2 * P) * kSkSlotBytes;
   SkParams q{};
   q.G = mtiles % 8 == 0 && P % 8 == 0 ? 8 : 1;
@@ -4146,29 +4281,18 @@ int forward_gemm(const ProjDesc* pd, int np, int64_t M, int64_t K, const void* x
   if (direct) {
     p.a = const_cast<uint16_t*>(static_cast<const uint16_t*>(x));
     for (int i = 0; i < si; ++i) p.seg[i].abase = 0;
-    if (sk) hipLaunchKernelGGL((gemm_latent_sk_kernel<false, true>), gsk, dim3(kGThreads), 0, s, p, q);
-    else hipLaunchKernelGGL((gemm_latent_kernel<false, true>), g1, dim3(kGThreads), lds, s, p);
+    if (sk) hipLaunchKernelGGL(gemm_latent_sk_kernel<true>, gsk, dim3(kGThreads), 0, s, p, q);
+    else hipLaunchKernelGGL(gemm_latent_kernel<true>, g1, dim3(kGThreads), lds, s, p);
   } else {
-    if (x_dtype == LBK_F32) hipLaunchKernelGGL((gemm_scale_kernel<float, true>), g0, dim3(kGThreads), 0, s, p);
-    else hipLaunchKernelGGL((gemm_scale_kernel<uint16_t, false>), g0, dim3(kGThreads), 0, s, p);
+    hipLaunchKernelGGL(gemm_scale_kernel<uint16_t>, g0, dim3(kGThreads), 0, s, p);
     rc = check_launch("gemm_scale_kernel");
     if (rc != LBK_OK) return rc;
-    if (split) {
-      if (sk) hipLaunchKernelGGL((gemm_latent_sk_kernel<true, false>), gsk, dim3(kGThreads), 0, s, p, q);
-      else hipLaunchKernelGGL((gemm_latent_kernel<true, false>), g1, dim3(kGThreads), lds, s, p);
-    } else {
-      if (sk) hipLaunchKernelGGL((gemm_latent_sk_kernel<false, false>), gsk, dim3(kGThreads), 0, s, p, q);
-      else hipLaunchKernelGGL((gemm_latent_kernel<false, false>), g1, dim3(kGThreads), lds, s, p);
-    }
+    if (sk) hipLaunchKernelGGL(gemm_latent_sk_kernel<false>, gsk, dim3(kGThreads), 0, s, p, q);
+    else hipLaunchKernelGGL(gemm_latent_kernel<false>, g1, dim3(kGThreads), lds, s, p);
   }
   rc = check_launch("gemm_latent_kernel");
   if (rc != LBK_OK) return rc;
-  if (split) {
-    if (y_dtype == LBK_F32) hipLaunchKernelGGL((gemm_expand_kernel<float, true>), g2, dim3(kGThreads), lds, s, p);
-    else hipLaunchKernelGGL((gemm_expand_kernel<uint16_t, true>), g2, dim3(kGThreads), lds, s, p);
-    return check_launch("gemm_expand_kernel");
-  }
-  // bf16 activations: 256-column tiles where they still give every CU two
+  // 256-column tiles where they still give every CU two
   // blocks (the stage ring allows two per CU); else 128-column tiles
   int ntw = 0;
   for (int q = 0; q < np; ++q) ntw += int(ceil_div(pd[q].N, 2 * kGB));
@@ -4182,8 +4306,8 @@ int forward_gemm(const ProjDesc* pd, int np, int64_t M, int64_t K, const void* x
     else hipLaunchKernelGGL((gemm_expand_wide_kernel<uint16_t>), gw, dim3(kGThreads), lds, s, p);
     return check_launch("gemm_expand_wide_kernel");
   }
-  if (y_dtype == LBK_F32) hipLaunchKernelGGL((gemm_expand_kernel<float, false>), g2, dim3(kGThreads), lds, s, p);
-  else hipLaunchKernelGGL((gemm_expand_kernel<uint16_t, false>), g2, dim3(kGThreads), lds, s, p);
+  if (y_dtype == LBK_F32) hipLaunchKernelGGL((gemm_expand_kernel<float>), g2, dim3(kGThreads), lds, s, p);
+  else hipLaunchKernelGGL((gemm_expand_kernel<uint16_t>), g2, dim3(kGThreads), lds, s, p);
   return check_launch("gemm_expand_kernel");
 }
 
@@ -4336,6 +4460,8 @@ int run_group(const ProjDesc* pd, int np, int64_t M, int64_t K, const void* x, i
     // one launch pair (each block takes one chunk's rows)
     return forward_mfma(pd, np, pl, M, K, x, x_dtype, in, y_dtype, workspace, s);
   }
+  if (pl.split && workspace_bytes >= sg_ws_bytes(pd, np, M, K))
+    return forward_split(pd, np, M, K, x, x_dtype, in, y_dtype, workspace, workspace_bytes, s);
   if (pl.chunk > 0) {
     // one launch pair per chunk (deterministic mode sizes its partials for
     // one chunk; or the rows' t does not fit the latent half at once)

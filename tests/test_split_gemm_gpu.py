@@ -1,0 +1,111 @@
+"""GPU: the split GEMM path (fp32 activations at more than 64 rows; 33-64 rows
+whose latent vectors do not fit the decode path's buffer) at the edges of its
+tiles, its k parts and its sign-word loads, against the oracle."""
+import numpy as np
+import pytest
+import torch
+
+import oracle.littlebit_oracle as O
+
+pytestmark = pytest.mark.gpu
+
+# hi + lo planes keep 16-17 mantissa bits of every product's activation
+# (2**-17 of its magnitude), as on the decode path
+TOL = 1e-3
+
+
+def _make(gpu, seed, M, K, specs, x_dtype, tile_v=True, offset=0):
+    from littlebit_amd import LittleBitBranch, LittleBitProjection, LittleBitProjectionGroup
+    from littlebit_amd.synthetic import make_branch
+    rng = np.random.Generator(np.random.PCG64(seed))
+    host = [[make_branch(rng, K, R, N) for R in ranks] for N, ranks in specs]
+    t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(gpu)  # noqa: E731
+    projs = [LittleBitProjection([LittleBitBranch(t(b.v_sign), t(b.u_sign), t(b.g), t(b.l), t(b.h)) for b in brs],
+                                 tile_v=tile_v) for brs in host]
+    buf = torch.zeros(M * K + offset, dtype=x_dtype, device=gpu)
+    x = buf[offset:].view(M, K)
+    x.copy_(torch.from_numpy(rng.standard_normal((M, K)).astype(np.float32)).to(gpu))
+    return host, LittleBitProjectionGroup(projs), x
+
+
+def _check(host, specs, K, x, outs, rows=None):
+    xu = x.float().cpu().numpy()
+    rows = np.arange(xu.shape[0]) if rows is None else rows
+    for (N, _), brs, y in zip(specs, host, outs):
+        ref = O.littlebit_forward(xu[rows], [b.as_dict() for b in brs], K, N)
+        err = O.rel_err(y.cpu().numpy()[rows], ref)
+        print(f"[split] M={xu.shape[0]} K={K} N={N} rel_err={err:.2e}", flush=True)
+        assert err <= TOL, (N, err)
+
+
+@pytest.mark.parametrize("M,K,specs", [
+    (65, 4096, [(4096, [205, 1843])]),              # k in parts, one row past two row tiles
+    (97, 1000, [(300, [127, 129])]),                # K off the word groups, ranks at a group's edge
+    (70, 33, [(1, [1, 5])]),                        # sign matrices of fewer than 4 words
+    (66, 32, [(3, [32]), (2, [70, 3])]),            # one-word rows, two projections
+    (128, 130, [(129, [128, 96]), (257, [31])]),    # last word partly used; one and two branches
+    (200, 260, [(4500, [40, 600])]),                # stage 2: 245 tiles of 32 x 128, ranks past 16 steps
+    (1100, 200, [(5000, [40, 600])]),               # stage 2 as 64 x 128 tiles, partial last tiles
+    (1100, 200, [(9000, [40, 601])]),               # stage 2 as 64 x 256 tiles, partial last tiles
+    (2049, 264, [(130, [205, 3000])]),              # stage 1 as 64-row tiles
+])
+def test_split_gemm_edges(gpu, M, K, specs):
+    host, grp, x = _make(gpu, 9100 + M, M, K, specs, torch.float32)
+    a = grp.forward(x)
+    b = grp.forward(x)
+    torch.cuda.synchronize()
+    rows = np.unique(np.r_[0:min(M, 40), max(0, M - 70):M])  # rows are independent
+    _check(host, specs, K, x, a, rows)
+    for u, v in zip(a, b):
+        assert torch.equal(u, v), "the split GEMM path repeats bit for bit"
+    host2, stored, x2 = _make(gpu, 9100 + M, M, K, specs, torch.float32, tile_v=False)
+    for u, v in zip(a, stored.forward(x2)):
+        assert torch.equal(u, v), "V as stored and V tiled hold the same signs"
+
+
+@pytest.mark.parametrize("M,x_dtype,offset", [(64, torch.float32, 0), (47, torch.bfloat16, 0), (100, torch.float32, 1)])
+def test_split_gemm_inputs(gpu, M, x_dtype, offset):
+    """RMSNorm, SiLU * up and plain inputs, residual in place, rows that take
+    the path because their latent vectors do not fit the decode buffer (two
+    projections of ranks 298 + 2686: 46 rows do not), misaligned x."""
+    K, specs = 520, [(1030, [298, 2686]), (514, [298, 2686])]
+    host, grp, x = _make(gpu, 9300 + M, M, K, specs, x_dtype, offset=offset)
+    gen = torch.Generator(device=gpu).manual_seed(M)
+    w = 1 + 0.1 * torch.randn(K, generator=gen, device=gpu)
+    up = torch.randn((M, K), generator=gen, device=gpu).to(x_dtype)
+    outs = [torch.randn((M, N), generator=gen, device=gpu) for N, _ in specs]
+    before = [o.clone() for o in outs]
+    grp.forward(x, outs=outs, out_dtype=torch.float32, residuals=outs, rms_weight=w)
+    xd = x.double()
+    h = (xd / torch.sqrt((xd * xd).mean(-1, keepdim=True) + 1e-6) * w.double()).float()
+    _check(host, specs, K, h, [o - r for o, r in zip(outs, before)])
+    outs = grp.forward(x, out_dtype=torch.float32, x_up=up)
+    _check(host, specs, K, (xd / (1 + torch.exp(-xd)) * up.double()).float(), outs)
+    _check(host, specs, K, x, grp.forward(x, out_dtype=torch.float32))
+
+
+def test_split_gemm_scale_ratios(gpu):
+    """Both branches share one accumulator set, rescaled by h0 / h1 between
+    them: ratios up to 2**+-60 with sums as large as their product with the
+    ratio still representable, zeros, and infinities stay where the formula
+    has them."""
+    M, K, N = 72, 256, 160
+    host, grp, x = _make(gpu, 9500, M, K, [(N, [64, 200])], torch.float32)
+    brs = host[0]
+    h0, h1 = brs[0].h, brs[1].h
+    for i in range(0, 120, 2):
+        h1[i] = h0[i] * np.float32(2.0 ** -(i // 2))
+        h0[i + 1] = h1[i + 1] * np.float32(2.0 ** -(i // 2))
+    h1[120:130] = 0.0
+    h0[130:140] = 0.0
+    big = np.float32(1e25)
+    grp.projections[0].branches[0].u1.copy_(torch.from_numpy(h0))
+    grp.projections[0].branches[1].u1.copy_(torch.from_numpy(h1))
+    for scale in (np.float32(1), big):
+        xs = x * float(scale)
+        y = grp.forward(xs)[0].cpu().numpy().astype(np.float64)
+        ref = O.littlebit_forward(xs.cpu().numpy(), [b.as_dict() for b in brs], K, N)
+        # per column: each column has its own scale
+        err = np.abs(y - ref).max(0) / np.abs(ref).max(0)
+        print(f"[split] ratios scale={scale:g} worst column {err.max():.2e}", flush=True)
+        assert np.isfinite(y).all() and err.max() <= TOL
