@@ -39,7 +39,7 @@
 extern "C" {
 #endif
 
-#define LBK_ABI_VERSION 9
+#define LBK_ABI_VERSION 10
 
 /* Element types of activations and outputs. */
 #define LBK_F32 0
@@ -300,6 +300,16 @@ int lbk_attention_batch(const float* q, const float* k, const float* v,
                         const int64_t* start_device, int64_t start,
                         const uint8_t* tree_mask, float scale, float* partial,
                         size_t partial_bytes, float* out, void* stream);
+
+/* The same for any number of new tokens n >= 1, causal, the start given by the
+ * host, in one launch without scratch (prompts: lbk_attention_batch is the
+ * faster one up to its 64 tokens).  start + n <= max_seq; q, k, v, the caches
+ * and out 16-byte aligned; out shares no memory with the others. */
+int lbk_attention_prefill(const float* q, const float* k, const float* v,
+                          float* k_cache, float* v_cache, int n, int heads,
+                          int kv_heads, int head_dim, int max_seq,
+                          int64_t start, float scale, float* out,
+                          void* stream);
 
 /* Expand packed signs to int8 {-1,+1}: out [rows, cols].
  * Replaces binary_unpacker (quantization/utils/binary_packer.py:54-97). */

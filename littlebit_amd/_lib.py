@@ -150,6 +150,11 @@ SIGNATURES = {
         [_VP, _VP, _VP, _VP, _VP, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, _VP, _I64,
          _VP, ctypes.c_float, _VP, ctypes.c_size_t, _VP, _VP],
     ),
+    "lbk_attention_prefill": (
+        ctypes.c_int,
+        [_VP, _VP, _VP, _VP, _VP, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, _I64,
+         ctypes.c_float, _VP, _VP],
+    ),
     "lbk_unpack_signs": (ctypes.c_int, [_VP, _I64, _I64, _VP, _VP]),
     "lbk_pack_signs": (ctypes.c_int, [_VP, _I64, _I64, _VP, _VP]),
     "lbk_repack_signs_to_i2": (ctypes.c_int, [_VP, _I64, _I64, _I64, _VP, _VP]),

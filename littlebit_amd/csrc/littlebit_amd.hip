@@ -3138,6 +3138,8 @@ __global__ __launch_bounds__(HD) void attn_batch_combine_kernel(AttnBatchParams 
   p.out[(size_t(qi) * p.heads + h) * HD + d] = merge_partials(pp, cstride, p.chunks, HD, d);
 }
 
+#include "attn_prefill.h"
+
 // ---------------------------------------------------------------------------
 // Q4_0 lm_head and argmax: the tail of the reference's generate_token
 // (patches/littlebit_cpu_optimized.cpp:2254-2317).  The weight is quantised
@@ -5136,6 +5138,49 @@ int lbk_attention_batch(const float* q, const float* k, const float* v, float* k
   if (head_dim == 128) hipLaunchKernelGGL(attn_batch_combine_kernel<128>, cgrid, dim3(128), 0, s, p);
   else hipLaunchKernelGGL(attn_batch_combine_kernel<64>, cgrid, dim3(64), 0, s, p);
   return check_launch("attn_batch_combine_kernel");
+}
+
+int lbk_attention_prefill(const float* q, const float* k, const float* v, float* k_cache, float* v_cache, int n,
+                          int heads, int kv_heads, int head_dim, int max_seq, int64_t start, float scale, float* out,
+                          void* stream) {
+  g_last_error[0] = '\0';
+  if (n < 1) return set_error(LBK_ERR_ARG, "n must be >= 1, got %d", n);
+  if (heads < 1 || kv_heads < 1 || heads % kv_heads != 0)
+    return set_error(LBK_ERR_ARG, "heads (%d) must be a positive multiple of kv_heads (%d)", heads, kv_heads);
+  if (head_dim != 64 && head_dim != 128) return set_error(LBK_ERR_ARG, "head_dim must be 64 or 128, got %d", head_dim);
+  if (max_seq < 1 || max_seq > (1 << 24)) return set_error(LBK_ERR_ARG, "max_seq out of range: %d", max_seq);
+  if (start < 0 || start + n > max_seq)
+    return set_error(LBK_ERR_ARG, "positions %lld .. %lld outside [0, %d)", (long long)start, (long long)(start + n - 1),
+                     max_seq);
+  if (!q || !k || !v || !k_cache || !v_cache || !out) return set_error(LBK_ERR_ARG, "NULL pointer");
+  for (const void* ptr : {static_cast<const void*>(q), static_cast<const void*>(k), static_cast<const void*>(v),
+                          static_cast<const void*>(k_cache), static_cast<const void*>(v_cache),
+                          static_cast<const void*>(out)})
+    if (!aligned16(ptr)) return set_error(LBK_ERR_ARG, "q, k, v, the caches and out must be 16-byte aligned");
+  const int64_t rows = int64_t(n) * (heads / kv_heads), tiles = ceil_div(rows, 32);
+  // the kernel's row numbers and in-tile byte offsets are 32-bit
+  if (rows > INT_MAX - 64 || tiles * kv_heads > INT_MAX || int64_t(kv_heads) * head_dim > (1 << 22))
+    return set_error(LBK_ERR_ARG, "%d tokens of %d heads (%d kv heads) are too many for one call", n, heads, kv_heads);
+  AttnPrefillParams p;
+  p.q = q;
+  p.k = k;
+  p.v = v;
+  p.kc = k_cache;
+  p.vc = v_cache;
+  p.out = out;
+  p.start = int(start);
+  p.N = n;
+  p.heads = heads;
+  p.kvh = kv_heads;
+  p.rep = heads / kv_heads;
+  p.max_seq = max_seq;
+  p.ntile = int(tiles);
+  p.scale = scale;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  const dim3 grid{unsigned(tiles * kv_heads), 1u, 1u};
+  if (head_dim == 128) hipLaunchKernelGGL(attn_prefill_kernel<128>, grid, dim3(256), 0, s, p);
+  else hipLaunchKernelGGL(attn_prefill_kernel<64>, grid, dim3(256), 0, s, p);
+  return check_launch("attn_prefill_kernel");
 }
 
 int lbk_q4_0_quantize(const float* w, int64_t rows, int64_t cols, uint8_t* qs, uint16_t* d, void* stream) {

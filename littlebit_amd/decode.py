@@ -143,8 +143,8 @@ class LittleBitDecoder:
         self.k_cache = torch.zeros(shape, dtype=torch.float32, device=dev)
         self.v_cache = torch.zeros(shape, dtype=torch.float32, device=dev)
         self.cache_pos = 0
-        # one-token steps and batches of up to 64 tokens use the HIP attention
-        # (head_dim 64 or 128)
+        # head_dim 64 or 128: the HIP attention (one token, batches of up to 64
+        # with a causal or tree mask, longer causal prompts)
         self._hip_attn = self.fuse and c.head_dim in (64, 128)
         if self._hip_attn:
             from . import _lib
@@ -175,6 +175,8 @@ class LittleBitDecoder:
             return self._attention_hip(q, k, v, kc, vc, start, pos_t)
         if 1 < N <= 64 and pos_t is None and self._hip_attn and length == start + N:
             return self._attention_batch_hip(q, k, v, kc, vc, start, tree_mask)
+        if N > 64 and tree_mask is None and pos_t is None and self._hip_attn and length == start + N:
+            return self._attention_prefill_hip(q, k, v, kc, vc, start)
         k3 = k.view(N, kvh, hd).transpose(0, 1)
         v3 = v.view(N, kvh, hd).transpose(0, 1)
         if pos_t is None:
@@ -259,6 +261,20 @@ class LittleBitDecoder:
             float(c.attn_scale), self._batch_part.data_ptr(), self._batch_part.numel() * 4, out.data_ptr(),
             torch.cuda.current_stream(q.device).cuda_stream)
         _lib.check(rc, "lbk_attention_batch")
+        return out
+
+    def _attention_prefill_hip(self, q, k, v, kc, vc, start: int):
+        """More than 64 new tokens (a prompt), causal, in one launch."""
+        from . import _lib
+        c = self.config
+        N = q.shape[0]
+        out = torch.empty((N, c.num_attention_heads * c.head_dim), dtype=torch.float32, device=q.device)
+        q, k, v = (t.to(torch.float32).contiguous() for t in (q, k, v))
+        rc = _lib.load().lbk_attention_prefill(
+            q.data_ptr(), k.data_ptr(), v.data_ptr(), kc.data_ptr(), vc.data_ptr(), N, c.num_attention_heads,
+            c.num_key_value_heads, c.head_dim, self.max_seq_len, int(start), float(c.attn_scale), out.data_ptr(),
+            torch.cuda.current_stream(q.device).cuda_stream)
+        _lib.check(rc, "lbk_attention_prefill")
         return out
 
     def forward_hidden(self, x: torch.Tensor, start: int, length: Optional[int] = None,
