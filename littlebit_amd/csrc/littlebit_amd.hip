@@ -3904,7 +3904,7 @@ bool t_fits(const ProjDesc* pd, int np, int64_t M) {
 // 32 rows that would run as 16-row chunks one after another take the split
 // GEMM path instead (64 rows of the target's q/k/v 178 -> 47 us, gate/up 310
 // -> 61 us), as long as the workspace holds its planes.
-Plan make_plan(const ProjDesc* pd, int np, int64_t M, int64_t K, bool allow_ks, bool det) {
+Plan compute_plan(const ProjDesc* pd, int np, int64_t M, int64_t K, bool allow_ks, bool det) {
   const Plan pl = plan_one(pd, np, M, K, allow_ks, det);
   const bool side_by_side = !det && t_fits(pd, np, M);
   if ((!pl.mfma || (M > 8 && side_by_side)) && M > 1 && M <= kMaxChunkedM) {
@@ -3921,6 +3921,43 @@ Plan make_plan(const ProjDesc* pd, int np, int64_t M, int64_t K, bool allow_ks, 
     }
   }
   return pl;
+}
+
+// The plan of a call's shapes.  A decoder asks for the same few shapes all
+// the time (a workspace query and a launch per call, 1-3 us of estimates for a
+// group at 8 rows), so each thread keeps the plans of up to 64 shapes: a
+// function of the values in the key alone, replaced when another shape falls
+// on the slot.
+Plan make_plan(const ProjDesc* pd, int np, int64_t M, int64_t K, bool allow_ks, bool det) {
+  struct Key {
+    int64_t v[3 + 4 * kMaxProj];
+  };
+  struct Slot {
+    Key key;
+    Plan plan;
+    bool used;
+  };
+  static thread_local Slot slots[64];
+  Key key;
+  memset(&key, 0, sizeof(key));
+  key.v[0] = M;
+  key.v[1] = K;
+  key.v[2] = np | (allow_ks ? 16 : 0) | (det ? 32 : 0);
+  uint64_t hash = (uint64_t(M) * 64 + uint64_t(key.v[2])) * 0x9E3779B97F4A7C15ull + uint64_t(K);
+  for (int q = 0; q < np; ++q) {
+    int64_t* v = key.v + 3 + 4 * q;
+    v[0] = pd[q].N;
+    v[1] = pd[q].nb;
+    for (int b = 0; b < pd[q].nb; ++b) v[2 + b] = pd[q].br[b].rank;
+    for (int i = 0; i < 4; ++i) hash = (hash ^ uint64_t(v[i])) * 0x9E3779B97F4A7C15ull;
+  }
+  Slot& s = slots[hash >> 58];
+  if (!s.used || memcmp(&s.key, &key, sizeof(key)) != 0) {
+    s.plan = compute_plan(pd, np, M, K, allow_ks, det);
+    s.key = key;
+    s.used = true;
+  }
+  return s.plan;
 }
 
 template <typename XT, int MT, int WPL>

@@ -46,7 +46,8 @@ from typing import Dict, List, Optional, Sequence, Tuple
 import torch
 import torch.nn.functional as F
 
-from .ops import LittleBitProjection, LittleBitProjectionGroup, PrivateWorkspace, private_workspace
+from .ops import (LittleBitProjection, LittleBitProjectionGroup, PrivateWorkspace, _raw_stream,
+                  private_workspace)
 from .runtime import load_runtime_checkpoint, runtime_projections
 
 __all__ = ["DecoderConfig", "LittleBitDecoder", "GPUDraftModel", "GPUTargetModel", "rms_norm"]
@@ -218,7 +219,7 @@ class LittleBitDecoder:
             q.data_ptr(), k.data_ptr(), v.data_ptr(), kc.data_ptr(), vc.data_ptr(), c.num_attention_heads,
             c.num_key_value_heads, c.head_dim, self.max_seq_len, None if pos_t is None else pos_t.data_ptr(),
             int(start), float(c.attn_scale), self._attn_part.data_ptr(), self._attn_part.numel() * 4, out.data_ptr(),
-            torch.cuda.current_stream(q.device).cuda_stream)
+            _raw_stream(q.device.index))
         _lib.check(rc, "lbk_attention_decode")
         return out
 
@@ -233,7 +234,7 @@ class LittleBitDecoder:
             q.data_ptr(), k.data_ptr(), v.data_ptr(), self.k_cache[li].data_ptr(), self.v_cache[li].data_ptr(),
             c.num_attention_heads, c.num_key_value_heads, c.head_dim, self.max_seq_len,
             None if pos_t is None else pos_t.data_ptr(), int(start), float(c.attn_scale), self._attn_part.data_ptr(),
-            self._attn_part.numel() * 4, None, torch.cuda.current_stream(q.device).cuda_stream)
+            self._attn_part.numel() * 4, None, _raw_stream(q.device.index))
         _lib.check(rc, "lbk_attention_decode")
         return AttentionPartials(self._attn_part, c.head_dim, self.max_seq_len, pos_t, int(start))
 
@@ -259,7 +260,7 @@ class LittleBitDecoder:
             c.num_key_value_heads, c.head_dim, self.max_seq_len, None if pos_t is None else pos_t.data_ptr(),
             int(start), None if tm is None else tm.data_ptr(),
             float(c.attn_scale), self._batch_part.data_ptr(), self._batch_part.numel() * 4, out.data_ptr(),
-            torch.cuda.current_stream(q.device).cuda_stream)
+            _raw_stream(q.device.index))
         _lib.check(rc, "lbk_attention_batch")
         return out
 
@@ -273,7 +274,7 @@ class LittleBitDecoder:
         rc = _lib.load().lbk_attention_prefill(
             q.data_ptr(), k.data_ptr(), v.data_ptr(), kc.data_ptr(), vc.data_ptr(), N, c.num_attention_heads,
             c.num_key_value_heads, c.head_dim, self.max_seq_len, int(start), float(c.attn_scale), out.data_ptr(),
-            torch.cuda.current_stream(q.device).cuda_stream)
+            _raw_stream(q.device.index))
         _lib.check(rc, "lbk_attention_prefill")
         return out
 

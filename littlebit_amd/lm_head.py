@@ -17,7 +17,7 @@ from typing import Optional
 import torch
 
 from . import _lib
-from .ops import _check, _require_cuda
+from .ops import _check, _raw_stream, _require_cuda
 
 
 class Q4LMHead:
@@ -67,7 +67,7 @@ class Q4LMHead:
             _require_cuda(logits, "logits")
             _check(logits.dtype == torch.float32 and logits.numel() == self.vocab, "logits must be float32 [vocab]")
         lib = _lib.load()
-        stream = torch.cuda.current_stream(self.device).cuda_stream
+        stream = _raw_stream(x.device.index)
         rc = lib.lbk_lm_head_q4_argmax(
             self.qs.data_ptr(), self.d.data_ptr(), self.vocab, self.hidden, x.data_ptr(),
             None if norm_weight is None else norm_weight.data_ptr(), float(eps),

@@ -292,7 +292,7 @@ class LittleBitLinear(nn.Linear):
     # forward (littlebit.py:95-121)
     # ------------------------------------------------------------------
     def _projection(self) -> LittleBitProjection:
-        if self._proj is not None and self._proj.device == self.U_packed.device:
+        if self._proj is not None and self._proj.device == self._buffers["U_packed"].device:
             return self._proj
         branches = []
         for branch in self._branches():

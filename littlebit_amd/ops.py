@@ -110,6 +110,11 @@ def deterministic(on: bool = True):
         set_deterministic(prev)
 
 
+# The handle of a device's current stream without the Stream object around it
+# (2 us a call, of the 8 that a one-row call spends in Python).
+_raw_stream = torch._C._cuda_getCurrentRawStream
+
+
 def _ws_key(device: torch.device, stream: int) -> Tuple[int, int]:
     return (device.index if device.index is not None else torch.cuda.current_device(), int(stream))
 
@@ -125,7 +130,7 @@ def workspace_for(device: torch.device, stream: int, nbytes: int) -> torch.Tenso
     priv = getattr(_override, "ws", None)
     if priv is not None:
         return priv.get(device, nbytes)
-    key = _ws_key(device, stream)
+    key = (device.index, stream) if device.index is not None else _ws_key(device, stream)
     ws = _workspaces.get(key)
     if ws is None or ws.numel() < nbytes:
         ws = torch.zeros(max(nbytes, 1 << 16), dtype=torch.uint8, device=device)
@@ -159,6 +164,25 @@ def _require_cuda(t: torch.Tensor, name: str) -> None:
     _check(isinstance(t, torch.Tensor), f"{name} must be a tensor")
     _check(t.is_cuda, f"{name} must be a GPU tensor (the HIP path has no CPU fallback)")
     _check(t.is_contiguous(), f"{name} must be contiguous")
+
+
+def _input_rows(x, in_features: int, device: torch.device):
+    """Checks of a call's input: (x as contiguous rows, their number, x's leading dimensions)."""
+    if not (isinstance(x, torch.Tensor) and x.is_cuda):
+        raise RuntimeError("input must be a GPU tensor")
+    if x.device != device:
+        raise RuntimeError("input must be on the factors' device")
+    if x.dtype not in _DTYPE_CODES:
+        raise RuntimeError(f"input dtype {x.dtype} unsupported (float32 or bfloat16)")
+    shape = x.shape
+    if not shape or shape[-1] != in_features:
+        raise RuntimeError(f"input last dimension {shape[-1] if shape else 'none'} != in_features {in_features}")
+    if len(shape) == 2 and x.is_contiguous():
+        return x, shape[0], (shape[0],)
+    x2 = x.reshape(-1, in_features)
+    if not x2.is_contiguous():
+        x2 = x2.contiguous()
+    return x2, x2.shape[0], tuple(shape[:-1])
 
 
 @dataclass
@@ -295,35 +319,27 @@ class LittleBitProjection:
                 self._group = LittleBitProjectionGroup([self])
             return self._group.forward(x, None if out is None else [out], out_dtype, rms_weight=rms_weight,
                                        rms_eps=rms_eps, x_up=x_up, residuals=[residual], attn=attn)[0]
-        _check(isinstance(x, torch.Tensor) and x.is_cuda, "input must be a GPU tensor")
-        _check(x.device == self.device, "input must be on the factors' device")
-        _check(x.dtype in _DTYPE_CODES, f"input dtype {x.dtype} unsupported (float32 or bfloat16)")
-        _check(x.shape[-1] == self.in_features,
-               f"input last dimension {x.shape[-1]} != in_features {self.in_features}")
-        lead = tuple(x.shape[:-1])
-        x2 = x.reshape(-1, self.in_features)
-        if not x2.is_contiguous():
-            x2 = x2.contiguous()
-        M = x2.shape[0]
+        x2, M, lead = _input_rows(x, self.in_features, self.device)
         odt = out_dtype or x.dtype
-        _check(odt in _DTYPE_CODES, f"output dtype {odt} unsupported")
+        ycode = _DTYPE_CODES.get(odt)
+        if ycode is None:
+            raise RuntimeError(f"output dtype {odt} unsupported")
         if out is None:
             out = torch.empty((*lead, self.out_features), dtype=odt, device=x.device)
-        else:
-            _check(out.is_cuda and out.is_contiguous() and out.dtype == odt
-                   and out.numel() == M * self.out_features, "out has the wrong shape, dtype or layout")
+        elif not (out.is_cuda and out.is_contiguous() and out.dtype == odt and out.numel() == M * self.out_features):
+            raise RuntimeError("out has the wrong shape, dtype or layout")
         if M == 0:
             return out
         lib = _lib.load()
-        stream = torch.cuda.current_stream(x.device).cuda_stream
-        need = self.workspace_bytes(M)
-        ws = workspace_for(x.device, stream, need)
+        stream = _raw_stream(self.device.index)
+        ws = workspace_for(x.device, stream, self.workspace_bytes(M))
         rc = lib.lbk_linear_forward(
             self._arr, len(self.branches), M, self.in_features, self.out_features,
             x2.data_ptr(), _DTYPE_CODES[x.dtype],
             self.bias.data_ptr() if self.bias is not None else None,
-            out.data_ptr(), _DTYPE_CODES[odt], ws.data_ptr(), ws.numel(), stream)
-        _call(rc, "lbk_linear_forward", x.device, stream)
+            out.data_ptr(), ycode, ws.data_ptr(), ws.numel(), stream)
+        if rc != _lib.LBK_OK:
+            _call(rc, "lbk_linear_forward", x.device, stream)
         return out
 
     __call__ = forward
@@ -394,17 +410,9 @@ class LittleBitProjectionGroup:
             inp = _lib.LbkInput(_lib.LBK_INPUT_ATTN_MERGE, None, 0.0, None, int(attn.head_dim), int(attn.max_seq),
                                 None if attn.pos is None else attn.pos.data_ptr(), int(attn.pos_host))
             return self._launch(x2, M, lead, odt, outs, inp, residuals)
-        _check(isinstance(x, torch.Tensor) and x.is_cuda, "input must be a GPU tensor")
-        _check(x.device == self.device, "input must be on the factors' device")
-        _check(x.dtype in _DTYPE_CODES, f"input dtype {x.dtype} unsupported (float32 or bfloat16)")
-        _check(x.shape[-1] == self.in_features,
-               f"input last dimension {x.shape[-1]} != in_features {self.in_features}")
-        _check(rms_weight is None or x_up is None, "rms_weight and x_up exclude each other")
-        lead = tuple(x.shape[:-1])
-        x2 = x.reshape(-1, self.in_features)
-        if not x2.is_contiguous():
-            x2 = x2.contiguous()
-        M = x2.shape[0]
+        if rms_weight is not None and x_up is not None:
+            raise RuntimeError("rms_weight and x_up exclude each other")
+        x2, M, lead = _input_rows(x, self.in_features, self.device)
         odt = out_dtype or x.dtype
         inp = None
         if rms_weight is not None:
@@ -419,32 +427,39 @@ class LittleBitProjectionGroup:
         return self._launch(x2, M, lead, odt, outs, inp, residuals)
 
     def _launch(self, x2, M, lead, odt, outs, inp, residuals) -> list:
-        _check(odt in _DTYPE_CODES, f"output dtype {odt} unsupported")
+        ycode = _DTYPE_CODES.get(odt)
+        if ycode is None:
+            raise RuntimeError(f"output dtype {odt} unsupported")
         if outs is None:
             outs = [torch.empty((*lead, p.out_features), dtype=odt, device=x2.device) for p in self.projections]
         else:
             _check(len(outs) == len(self.projections), "one output per projection")
             for o, p in zip(outs, self.projections):
-                _check(o.is_cuda and o.is_contiguous() and o.dtype == odt and o.numel() == M * p.out_features,
-                       "an output has the wrong shape, dtype or layout")
+                if not (o.is_cuda and o.is_contiguous() and o.dtype == odt and o.numel() == M * p.out_features):
+                    raise RuntimeError("an output has the wrong shape, dtype or layout")
         if M == 0:
             return list(outs)
-        keep = []
+        arr = self._arr
         for i, o in enumerate(outs):
-            self._arr[i].y = o.data_ptr()
+            d = arr[i]
+            d.y = o.data_ptr()
             r = None if residuals is None else residuals[i]
-            if r is not None:
-                _require_cuda(r, f"residuals[{i}]")
-                _check(r.dtype == torch.float32 and r.numel() == o.numel(), "a residual must be float32 like its output")
-                keep.append(r)
-            self._arr[i].residual = None if r is None else r.data_ptr()
+            if r is None:
+                d.residual = None
+                continue
+            if r is not o:  # an output was checked above
+                _require_cuda(r, "residual")
+            if r.dtype != torch.float32 or r.numel() != o.numel():
+                raise RuntimeError("a residual must be float32 like its output")
+            d.residual = r.data_ptr()
         lib = _lib.load()
-        stream = torch.cuda.current_stream(x2.device).cuda_stream
+        stream = _raw_stream(self.device.index)
         ws = workspace_for(x2.device, stream, self.workspace_bytes(M))
-        rc = lib.lbk_group_forward_ex(self._arr, len(self.projections), M, self.in_features, x2.data_ptr(),
-                                      _DTYPE_CODES[x2.dtype], ctypes.byref(inp) if inp is not None else None,
-                                      _DTYPE_CODES[odt], ws.data_ptr(), ws.numel(), stream)
-        _call(rc, "lbk_group_forward_ex", x2.device, stream)
+        rc = lib.lbk_group_forward_ex(arr, len(self.projections), M, self.in_features, x2.data_ptr(),
+                                      _DTYPE_CODES[x2.dtype], None if inp is None else ctypes.byref(inp),
+                                      ycode, ws.data_ptr(), ws.numel(), stream)
+        if rc != _lib.LBK_OK:
+            _call(rc, "lbk_group_forward_ex", x2.device, stream)
         return list(outs)
 
     __call__ = forward
@@ -591,10 +606,11 @@ class LittleBitChain:
         the results are in the links' output tensors."""
         ptr = self._set_input(x, attn, x_up)
         lib = _lib.load()
-        stream = torch.cuda.current_stream(self.device).cuda_stream
+        stream = _raw_stream(self.device.index)
         ws = workspace_for(self.device, stream, self._ws_bytes)
         rc = lib.lbk_chain_forward(self._arr, len(self.links), ptr, ws.data_ptr(), ws.numel(), stream)
-        _call(rc, "lbk_chain_forward", self.device, stream)
+        if rc != _lib.LBK_OK:
+            _call(rc, "lbk_chain_forward", self.device, stream)
 
     __call__ = forward
 
