@@ -30,11 +30,8 @@
 //                       h0*y0 + h1*y1 + bias (one slice) or adds h0*y0 +
 //                       h1*y1 to y with fp32 atomics (several slices; the
 //                       latent kernel has set y = bias + residual).
-// GEMM path (M > 64, or operands too large for the decode path's LDS), bf16
-// activations: gemm_scale_kernel (bf16 g*x, when x cannot be read as it is) /
-//   gemm_latent_kernel (or its stream-K form) / gemm_expand_kernel (or its
-//   128 x 256 tile form), tiled on v_mfma_f32_32x32x16_bf16.  fp32
-//   activations: the kernels of split_gemm.h.
+// GEMM path (M > 64, or operands too large for the decode path's LDS): the
+// kernels of sign_gemm.h, tiled on v_mfma_f32_32x32x16_bf16.
 //
 // Splitting fp32 activations into bf16 hi + lo keeps the product error near
 // 2^-17 relative: +-1 is exact in bf16 and the MFMA accumulates in fp32.
@@ -74,8 +71,6 @@ constexpr int kMaxBlockLds = 159 * 1024;       // static + dynamic LDS of one bl
 constexpr int kRowBlock = 64;                  // latent rows per latent_mfma block
 constexpr int kMaxMfmaM = 16;                  // MFMA path handles M <= 16
 constexpr int kCounterSlots = 1024;            // counters at the workspace start
-constexpr float kTinyH = 1e-30f;               // |h1| below this: no h0 / h1 rescale (it could overflow)
-constexpr float kMaxHRatio = 1099511627776.f;  // 2^40: |h0 / h1| above this drops branch 1 (wide stage 2)
 constexpr size_t kCounterBytes = kCounterSlots * sizeof(uint32_t);
 
 // Encoding of s_waitcnt vmcnt(n) lgkmcnt(0) on gfx9 (expcnt left alone).
@@ -103,13 +98,6 @@ __device__ __forceinline__ uint16_t f32_to_bf16(float f) {
   return uint16_t(u >> 16);
 }
 __device__ __forceinline__ float bf16_to_f32(uint16_t b) { return __uint_as_float(uint32_t(b) << 16); }
-
-// Wide stage 2 keeps branch 1 of a column (rescaling acc by h0 / h1) unless
-// h1 is zero or denormal, or |h0 / h1| > 2^40 (the rescaled acc could
-// overflow, while h1's term is negligible there).
-__device__ __forceinline__ bool use_branch1(float h0, float h1) {
-  return fabsf(h1) >= kTinyH && fabsf(h0) <= fabsf(h1) * kMaxHRatio;
-}
 
 __device__ __forceinline__ void store_out(float* y, size_t i, float v) { y[i] = v; }
 __device__ __forceinline__ void store_out(uint16_t* y, size_t i, float v) { y[i] = f32_to_bf16(v); }
@@ -1944,656 +1932,9 @@ __global__ __launch_bounds__(W * kWave) void chain_mfma_kernel(ChainParams cp) {
 }
 
 // ---------------------------------------------------------------------------
-// GEMM path on bf16 activations (M > 64, and shapes the decode path cannot
-// stage in LDS; fp32 activations: split_gemm.h): a tiled sign-GEMM on
-// v_mfma_f32_32x32x16_bf16, three launches per call.
-//   prologue  A_s[m, k] = g_s[k] * x[m, k] per branch s, as bf16, k padded
-//             with zeros to a multiple of 64
-//   stage 1   T_s[m, r] = l_s[r] * sum_k sV_s[r, k] * A_s[m, k], as bf16
-//   stage 2   y[m, n] = bias[n] + sum_b h_b[n] * sum_r sU_b[n, r] * T_b[m, r]
-// One bf16 plane each: the precision of the reference's bf16 forward
-// (littlebit.py:116-121).
-// Stages 1 and 2: block tile 128 (m) x 128 (columns: latent rows in stage
-// 1, outputs in stage 2), 4 waves of 64 x 64 (2 x 2 MFMA tiles), k-steps of
-// 64.  A tiles go from global memory straight to LDS through a 4-stage ring
-// (see gemm_mainloop); the +-1 B operand is expanded in registers from the
-// sign words of the lane's column (staged in LDS by the block): for 16-k
-// sub-step s, lane l (column l % 32, k 8*(l/32) .. +8 of the 32x32x16
-// operand) takes byte 2*(s%2) + l/32 of word s/2 of the step.
+// GEMM path
 // ---------------------------------------------------------------------------
-constexpr int kGB = 128;             // block tile (m and columns)
-constexpr int kGK = 64;              // k per step (two sign words per column)
-constexpr int kGThreads = 256;
-
 typedef float f32x16 __attribute__((ext_vector_type(16)));
-
-struct GemmSeg {      // stage-1 operands of one branch
-  const uint32_t* V;  // [R, KW]
-  const float* g;     // [K]
-  const float* l;     // [R]
-  int R;
-  int RP;             // T row length: R rounded up to kGB
-  int nt0;            // first column tile of the segment
-  int64_t abase;      // offset of the segment's [M][Kp] block in an A plane
-  int64_t tbase;      // offset of the segment's [M][RP] block in a T plane
-};
-
-struct GemmProj {     // stage-2 operands of one projection
-  const uint32_t* U[2];
-  const float* h[2];
-  const float* bias;
-  const float* res;   // [M, N] fp32 added to y, or null (may alias y)
-  void* y;
-  int RW[2];          // words per U row
-  int RP[2];
-  int64_t tbase[2];
-  int nb;
-  int N;
-  int nt0;            // first column tile of the projection
-};
-
-struct GemmParams {
-  GemmSeg seg[kMaxSeg];
-  GemmProj proj[kMaxProj];
-  int nseg, nproj;
-  int M, K, KW;
-  int Kp;             // K rounded up to kGK
-  int xvec;           // x rows (x1, rms weight) and every g allow 16-byte loads
-  int xmode;          // LBK_INPUT_* (see load_input8)
-  const void* x;
-  const void* x1;
-  const float* nw;
-  float eps;
-  uint16_t* a;        // A
-  uint16_t* t;        // T
-};
-
-// Prologue.  grid = (M, segments), 256 threads; thread handles 8-k chunks.
-// The input mode (RMSNorm, SiLU * up) is applied here, as in load_input8.
-template <typename XT>
-__global__ __launch_bounds__(kGThreads) void gemm_scale_kernel(GemmParams p) {
-  const int m = int(blockIdx.x);
-  const GemmSeg& S = p.seg[__builtin_amdgcn_readfirstlane(int(blockIdx.y))];
-  const XT* __restrict__ xr = static_cast<const XT*>(p.x) + int64_t(m) * p.K;
-  const XT* __restrict__ ur = p.x1 ? static_cast<const XT*>(p.x1) + int64_t(m) * p.K : xr;
-  const float* __restrict__ g = S.g;
-  const int tid = int(threadIdx.x);
-  float rsm = 1.f;
-  if (p.xmode == LBK_INPUT_RMSNORM) {
-    __shared__ float rs[1];
-    __shared__ float rscratch[kGThreads / 64];
-    rms_scales<XT, 1, kGThreads>(xr, 1, p.K, p.eps, rs, rscratch, tid);
-    rsm = rs[0];
-  }
-  uint16_t* __restrict__ hi = p.a + S.abase + int64_t(m) * p.Kp;
-  for (int k = 8 * tid; k < p.Kp; k += 8 * kGThreads) {
-    float v[8];
-    if (p.xvec && k + 8 <= p.K) {
-      float gv[8];
-      load8(xr + k, v);
-      load8(g + k, gv);
-      if (p.xmode == LBK_INPUT_RMSNORM) {
-        float wv[8];
-        load8(p.nw + k, wv);
-#pragma unroll
-        for (int i = 0; i < 8; ++i) gv[i] *= wv[i] * rsm;
-      } else if (p.xmode == LBK_INPUT_SILU_MUL) {
-        float uv[8];
-        load8(ur + k, uv);
-#pragma unroll
-        for (int i = 0; i < 8; ++i) v[i] = silu_f(v[i]) * uv[i];
-      }
-#pragma unroll
-      for (int i = 0; i < 8; ++i) v[i] *= gv[i];
-    } else {
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        float e = 0.f;
-        if (k + i < p.K) {
-          const float xv = to_f32(xr[k + i]);
-          e = xv * g[k + i];
-          if (p.xmode == LBK_INPUT_RMSNORM) e *= p.nw[k + i] * rsm;
-          else if (p.xmode == LBK_INPUT_SILU_MUL) e = silu_f(xv) * to_f32(ur[k + i]) * g[k + i];
-        }
-        v[i] = e;
-      }
-    }
-    u32x4 h;
-#pragma unroll
-    for (int d = 0; d < 4; ++d) h[d] = uint32_t(f32_to_bf16(v[2 * d])) | (uint32_t(f32_to_bf16(v[2 * d + 1])) << 16);
-    *reinterpret_cast<u32x4*>(hi + k) = h;
-  }
-}
-
-// acc[i][j] += A[m0 + gemm_row(wm, i) + .., :64*nks] . S[:64*nks, c0 + gemm_col<NJ>(wn, j) + ..]
-// S[k, c] = sign bit k of row c of W (ldw words per row, zero past it);
-// step ks reads words 2*ks and 2*ks + 1.  The block covers 128 rows of A and
-// BN = 128 or 256 columns (wide: each staged A tile serves twice the
-// columns), its 4 waves laid out as below.
-//
-// A tiles (128 rows x 64 k per plane, rows past M repeat row M - 1) go from
-// global memory straight to LDS (global_load_lds_dwordx4) through a ring of
-// kGStages stages, issued kGStages - 1 steps ahead; each stage is its own
-// __shared__ array so that the compiler can tell which load fills which
-// stage.  Rows are 128 bytes, 16-byte chunk c of row r stored at chunk
-// c ^ swz(r), swz(r) = (r ^ (r >> 3)) & 7: the LDS serves a ds_read_b128 16
-// lanes (256 bytes, all 64 banks) at a time, and the 16 rows of such a group
-// -- 8 of each row parity, at the same offset mod 256 -- read 16 distinct
-// 16-byte bank groups (with c ^ (r & 7), rows r and r + 8 collided).
-//
-// The sign words of a step (2 per column, BN columns) are fetched by the
-// whole block, BN / 128 words per thread (columns 128 u + tid / 2, word
-// tid % 2), and written to one of two LDS buffers ([column][2 words]) from
-// which every lane of the step reads its columns' pair (8 bytes).  A lane fetching
-// its own columns' words instead costs 16 loads per block and step, each
-// touching 32 cache lines, and the two wave rows fetch the same words.
-//
-// With GB (stage 1 on bf16 activations taken as they are) the B operand is
-// +-g[k] instead of +-1: the 64 g values of a step are staged beside its
-// sign words, as bf16, in one of two 128-byte buffers (each wave fetches
-// them, wave 0 writes them), and each 16-k sub-step reads its 8 values.
-// In wide tiles (BN = 256) with h given (the second branch of stage 2, h0 the
-// first branch's row scale) it is +-1 where the lane's column c keeps
-// branch 1 (use_branch1(h0[c], h[c])) and 0 elsewhere; both branches run
-// the same instantiation, so they share one stage ring.
-//
-// fill(f) issues the DMA of step f and the sign word (and g) of step f + 1.  Every
-// fill issues the same loads on every path; before step ks every wave waits
-// (vmcnt) until only the two newer fills' loads are outstanding -- vector
-// loads complete in order, so fill(ks) has landed: stage ks is complete and
-// the sign word of step ks + 1 is in the register that step ks writes to LDS
-// (masked to zero past the row or the matrix) -- and a barrier makes the
-// tile, and the words step ks - 1 wrote, visible; fill(ks + 3) then refills
-// the stage and the register that step ks - 1 used.  Ends with a barrier.
-[[maybe_unused]] constexpr int kGStages = 4;  // the ring's stages (one __shared__ array each)
-
-// Wave layout of a GEMM block: kGWM waves along m, kGWN along the columns;
-// a wave holds kGMI x NJ tiles of 32 x 32 (NJ = BN / (32 kGWN)).  The B
-// operand is expanded in registers from the sign words, once per wave for
-// each of its column tiles, and feeds the kGMI MFMAs of that column; each A
-// fragment read from LDS feeds NJ.  Tall wave tiles (kGWM = 1: all 128 rows,
-// 4 x 1 tiles at BN = 128, 4 x 2 at BN = 256) expand each sign once per
-// block, half the VALU per MFMA of 2 x 2 waves, and read each A fragment for
-// NJ MFMAs instead of 2 NJ: measured, MFMAs fed from LDS lose about 1 % at
-// one fragment per MFMA, while VALU beyond about 4 per MFMA stalls the MFMA
-// pipe (bench.py --only issue).
-#ifndef LBK_GEMM_WM
-#define LBK_GEMM_WM 1
-#endif
-constexpr int kGWM = LBK_GEMM_WM;
-constexpr int kGWN = 4 / kGWM;
-constexpr int kGMI = kGB / (32 * kGWM);
-static_assert(kGWM == 1 || kGWM == 2, "wave layouts 1 x 4 and 2 x 2");
-template <int BN>
-constexpr int gemm_nj() {
-  return BN / (32 * kGWN);
-}
-__device__ __forceinline__ int gemm_row(int wm, int i) { return 32 * kGMI * wm + 32 * i; }
-template <int NJ>
-__device__ __forceinline__ int gemm_col(int wn, int j) {
-  return 32 * NJ * wn + 32 * j;
-}
-__device__ __forceinline__ int gemm_wm(int wave) { return kGWM == 1 ? 0 : wave >> 1; }
-__device__ __forceinline__ int gemm_wn(int wave) { return kGWM == 1 ? wave : wave & 1; }
-
-template <bool GB = false, int BN = 128>
-__device__ __forceinline__ void gemm_mainloop(const uint16_t* __restrict__ A, int64_t lda, int M,
-                                              int m0, const uint32_t* __restrict__ W, int ldw, int ncols, int c0,
-                                              int nks, f32x16 (&acc)[kGMI][gemm_nj<BN>()], int tid,
-                                              const float* __restrict__ g = nullptr, int kbase = 0,
-                                              const float* __restrict__ h = nullptr,
-                                              const float* __restrict__ h0 = nullptr) {
-  static_assert(BN == 128 || BN == 256, "blocks of 128 or 256 columns");
-  static_assert(BN == 128 || !GB, "wide tiles carry no g in the B operand");
-  constexpr int NJ = gemm_nj<BN>();
-  typedef __attribute__((address_space(3))) void* lds_ptr_t;
-  typedef __attribute__((address_space(1))) void* glb_ptr_t;
-  constexpr int NW = BN / 128;              // sign words per thread and step
-  constexpr int TILE = kGB * kGK;           // elements per stage
-  constexpr int LOADS_PER_FILL = 4 + NW + (GB ? 1 : 0);  // global_load_lds, sign words, g; per wave
-  __shared__ __attribute__((aligned(16))) uint16_t st0[TILE];
-  __shared__ __attribute__((aligned(16))) uint16_t st1[TILE];
-  __shared__ __attribute__((aligned(16))) uint16_t st2[TILE];
-  __shared__ __attribute__((aligned(16))) uint16_t st3[TILE];
-  __shared__ __attribute__((aligned(16))) uint32_t sw[2][2 * BN];
-  __shared__ __attribute__((aligned(16))) uint16_t gb[2][kGK];
-  const int lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = gemm_wm(wave), wn = gemm_wn(wave);
-  const int lr = lane & 31, lh = lane >> 5;
-  // Steps are numbered from kbase (the first k-step of the range, 64 k
-  // each); step st of the range is k-step kbase + st of the matrices.
-  // this thread's sign words of a step: word 2 * step + (tid & 1) of
-  // columns c0 + 128 u + tid / 2, stored at sw[.][2 * (128 u + tid / 2) + tid % 2]
-  const int sodd = tid & 1;
-  uint32_t smask[NW];
-  const uint32_t* __restrict__ srow[NW];
-#pragma unroll
-  for (int u = 0; u < NW; ++u) {
-    const int scol = c0 + 128 * u + (tid >> 1);
-    smask[u] = scol < ncols ? ~0u : 0u;
-    srow[u] = W + int64_t(scol < ncols ? scol : 0) * ldw;
-  }
-  struct Words {
-    uint32_t v[NW];
-  };
-  auto word_at = [&](int st) {
-    Words w;
-#pragma unroll
-    for (int u = 0; u < NW; ++u) w.v[u] = srow[u][min(2 * (kbase + st) + sodd, ldw - 1)];
-    return w;
-  };
-  // The empty asm pins each register's first use to its step: without it
-  // the compiler hoists the masking of later steps' words into this one and
-  // waits there for every outstanding load (vmcnt(0)), DMAs included.
-  auto put_word = [&](int st, Words raw) {
-#pragma unroll
-    for (int u = 0; u < NW; ++u) {
-      uint32_t r = raw.v[u];
-      asm volatile("" : "+v"(r));
-      sw[st & 1][256 * u + tid] = 2 * (kbase + st) + sodd < ldw ? r & smask[u] : 0u;
-    }
-  };
-  // wide tiles: the +-1 pair of the lane's column in subtile j, or 0 where
-  // h is given and the column drops branch 1 (columns past ncols have zero
-  // sign words)
-  uint32_t hv[NJ];
-  if constexpr (BN == 256) {
-#pragma unroll
-    for (int j = 0; j < NJ; ++j) {
-      const int n = min(c0 + gemm_col<NJ>(wn, j) + lr, ncols - 1);
-      hv[j] = !h || use_branch1(h0[n], h[n]) ? 0x3F803F80u : 0u;
-    }
-  }
-  // g of step st, lane's k (clamped: steps past the last are never read)
-  const int kmax = (kbase + nks) * kGK - 1;
-  auto g_at = [&](int st) { return GB ? g[min((kbase + st) * kGK + lane, kmax)] : 0.f; };
-  auto put_g = [&](int st, float v) {
-    if constexpr (GB) {
-      asm volatile("" : "+v"(v));
-      if (wave == 0) gb[st & 1][lane] = f32_to_bf16(v);
-    }
-  };
-  // this lane's source rows and chunks for its 4 DMA slots of a stage
-  const uint16_t* src[4];
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const int slot = (wave * 4 + j) * 64 + lane;
-    const int row = slot >> 3, c = (slot & 7) ^ ((row ^ (row >> 3)) & 7);
-    src[j] = A + int64_t(min(m0 + row, M - 1)) * lda + 8 * c;
-  }
-  auto issue = [&](int ks, uint16_t* st) {
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      uint16_t* dst = st + (wave * 4 + j) * 512;
-      __builtin_amdgcn_global_load_lds((glb_ptr_t)(src[j] + int64_t(kbase + ks) * kGK), (lds_ptr_t)dst, 16, 0, 0);
-    }
-  };
-  uint32_t kmask = 0x80008000u, kone = 0x3F803F80u;
-  asm volatile("" : "+v"(kmask), "+v"(kone));
-  auto compute = [&](int ks, const uint16_t* a) {
-    u32x4 gk[4];
-    if constexpr (GB) {
-#pragma unroll
-      for (int s = 0; s < 4; ++s) gk[s] = *reinterpret_cast<const u32x4*>(&gb[ks & 1][16 * s + 8 * lh]);
-    }
-    uint32_t w[NJ][2];
-#pragma unroll
-    for (int j = 0; j < NJ; ++j) {
-      const uint2 pr = *reinterpret_cast<const uint2*>(&sw[ks & 1][2 * (gemm_col<NJ>(wn, j) + lr)]);
-      w[j][0] = pr.x;
-      w[j][1] = pr.y;
-    }
-#pragma unroll
-    for (int s = 0; s < 4; ++s) {
-      bf16x8 b[NJ];
-#pragma unroll
-      for (int j = 0; j < NJ; ++j)
-        b[j] = GB   ? signs_times_bf16x8(w[j][s >> 1] >> (8 * lh), 2 * (s & 1), kmask, gk[s])
-               : BN == 256 ? signs_times_bf16x8(w[j][s >> 1] >> (8 * lh), 2 * (s & 1), kmask,
-                                               u32x4{hv[j], hv[j], hv[j], hv[j]})
-                    : signs_to_bf16x8(w[j][s >> 1] >> (8 * lh), 2 * (s & 1), kmask, kone);
-#pragma unroll
-      for (int i = 0; i < kGMI; ++i) {
-        const int r = gemm_row(wm, i) + lr;
-        const int off = r * kGK + (((2 * s + lh) ^ ((r ^ (r >> 3)) & 7)) << 3);
-        const bf16x8 ah = *reinterpret_cast<const bf16x8*>(a + off);
-#pragma unroll
-        for (int j = 0; j < NJ; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah, b[j], acc[i][j], 0, 0, 0);
-      }
-    }
-  };
-  // Past the last step a fill repeats step nks - 1's DMA into a stage nothing
-  // reads again (and a clamped word nothing reads), so exactly two fills'
-  // loads are always newer than fill(ks) at step ks.
-  auto fill = [&](int f, uint16_t* st, Words& w, float& gv) {
-    w = word_at(f + 1);
-    gv = g_at(f + 1);
-    issue(min(f, nks - 1), st);
-  };
-  // The memory clobbers keep LDS accesses from being moved across the
-  // barrier; the waitcnt and the barrier also delimit the scheduler's
-  // regions, so fills ks + 1 and ks + 2 issue all their loads after fill ks.
-  auto step = [&](int ks, const uint16_t* cur, Words wcur, float gcur, uint16_t* nxt, Words& wnxt,
-                  float& gnxt) {
-    __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(2 * LOADS_PER_FILL));
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-    put_word(ks + 1, wcur);
-    put_g(ks + 1, gcur);
-    fill(ks + 3, nxt, wnxt, gnxt);
-    compute(ks, cur);
-  };
-  put_word(0, word_at(0));
-  put_g(0, g_at(0));
-  Words w0, w1, w2, w3;
-  float g0, g1, g2, g3;
-  fill(0, st0, w0, g0);
-  __builtin_amdgcn_sched_barrier(0);
-  fill(1, st1, w1, g1);
-  __builtin_amdgcn_sched_barrier(0);
-  fill(2, st2, w2, g2);
-  __builtin_amdgcn_sched_barrier(0);
-  // whole rounds of the ring, then the remaining steps: every path into the
-  // loop header has issued the same loads
-  int ks = 0;
-  for (; ks + 4 <= nks; ks += 4) {
-    step(ks, st0, w0, g0, st3, w3, g3);
-    step(ks + 1, st1, w1, g1, st0, w0, g0);
-    step(ks + 2, st2, w2, g2, st1, w1, g1);
-    step(ks + 3, st3, w3, g3, st2, w2, g2);
-  }
-  if (ks < nks) step(ks, st0, w0, g0, st3, w3, g3);
-  if (ks + 1 < nks) step(ks + 1, st1, w1, g1, st0, w0, g0);
-  if (ks + 2 < nks) step(ks + 2, st2, w2, g2, st1, w1, g1);
-  __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(0));
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
-}
-
-// Stage 1 epilogue: T rows of the tile (m0, c0) of segment G, l-scaled.
-constexpr int kGNJ = gemm_nj<kGB>();  // column tiles per wave of a 128-column block
-
-__device__ __forceinline__ void latent_store(const GemmParams& p, const GemmSeg& G, int m0, int c0,
-                                             const f32x16 (&acc)[kGMI][kGNJ], int tid) {
-  const int lane = tid & 63, wave = tid >> 6;
-  const int wm = gemm_wm(wave), wn = gemm_wn(wave);
-  const int lr = lane & 31, lh = lane >> 5;
-  uint16_t* __restrict__ T = p.t + G.tbase;
-#pragma unroll
-  for (int j = 0; j < kGNJ; ++j) {
-    const int r = c0 + gemm_col<kGNJ>(wn, j) + lr;  // < RP; rows R <= r < RP are written as zeros
-    const float lv = r < G.R ? G.l[r] : 0.f;
-#pragma unroll
-    for (int i = 0; i < kGMI; ++i)
-#pragma unroll
-      for (int q = 0; q < 16; ++q) {
-        const int m = m0 + gemm_row(wm, i) + 8 * (q >> 2) + 4 * lh + (q & 3);
-        if (m < p.M) {
-          const int64_t o = int64_t(m) * G.RP + r;
-          const float v = lv * acc[i][j][q];
-          T[o] = f32_to_bf16(v);
-        }
-      }
-  }
-}
-
-__device__ __forceinline__ int latent_segment(const GemmParams& p, int nt) {
-  int si = 0;
-#pragma unroll
-  for (int i = 1; i < kMaxSeg; ++i) si += (i < p.nseg && nt >= p.seg[i].nt0) ? 1 : 0;
-  return __builtin_amdgcn_readfirstlane(si);
-}
-
-// Stage 1.  grid = (m-tiles, column tiles of all segments), 256 threads.
-// GB: A is the bf16 input itself (every segment's abase 0, rows of Kp = K)
-// and g goes into the B operand.
-template <bool GB>
-__global__ __launch_bounds__(kGThreads) void gemm_latent_kernel(GemmParams p) {
-  const int tid = int(threadIdx.x);
-  const int nt = int(blockIdx.y);
-  const GemmSeg& G = p.seg[latent_segment(p, nt)];
-  const int m0 = int(blockIdx.x) * kGB;
-  const int c0 = (nt - G.nt0) * kGB;
-  f32x16 acc[kGMI][kGNJ];
-#pragma unroll
-  for (int i = 0; i < kGMI; ++i)
-#pragma unroll
-    for (int j = 0; j < kGNJ; ++j) acc[i][j] = f32x16{};
-  gemm_mainloop<GB>(p.a + G.abase, p.Kp, p.M, m0, G.V, p.KW, G.R, c0, p.Kp / kGK, acc, tid, G.g);
-  latent_store(p, G, m0, c0, acc, tid);
-}
-
-// Stage 1, stream-K form: when the tiles do not fill the CUs' block slots
-// evenly (e.g. 272 tiles for 512 slots), resident blocks share the (tile,
-// k-step) iterations evenly instead.  The blocks form G groups (G = 8 when
-// the m-tiles divide by 8, else 1); group x = b % G takes the tiles of
-// m-tiles x, x + G, ... -- blocks are dealt to the 8 XCDs in turn, so each
-// XCD's L2 holds the rows of A of two m-tiles (at M = 2048), as in the
-// whole-tile grid -- and block b of the group's P blocks (b = blockIdx / G)
-// takes its iterations [b W / P, (b + 1) W / P), W = the group's tiles *
-// nks, tiles in m-major order.  A tile cut between blocks is
-// summed by its last part: every part stores its fp32 accumulators in its
-// block's slot (0: the part starts inside the tile, 1: it starts at the
-// tile's first step) and adds its step count to the tile's counter (indexed
-// by the first block of the tile: each block is the first of at most one cut
-// tile); the part whose count completes the tile sums all the parts' slots
-// in block order (the same sum on every run), zeroes the counter again and
-// stores T.  No part waits for another.
-// Partial tiles move through agent-scope stores and loads (sc1: written
-// through to, and read from, the point where all XCDs' L2s agree), ordered
-// by vmcnt(0) before the counter's atomic; fences would do the same by
-// writing back and invalidating whole L2s, which cost more than the tiles.
-struct SkParams {
-  int P;             // blocks per group
-  int G;             // groups (grid = G * P blocks)
-  int NT;            // column tiles over all segments
-  int nks;           // k-steps per tile
-  int64_t W;         // iterations per group: m-tiles / G * NT * nks
-  float* part;       // [G * P][2][64 * kGThreads] fp32 partial tiles
-  uint32_t* cnt;     // [G * P] step counters, zero between calls
-};
-
-__device__ __forceinline__ int64_t sk_start(int b, const SkParams& q) { return int64_t(b) * q.W / q.P; }
-// the block whose range holds iteration i: the largest b with sk_start(b) <= i
-__device__ __forceinline__ int sk_block(int64_t i, const SkParams& q) { return int(((i + 1) * q.P - 1) / q.W); }
-
-// Two blocks per CU (the sk_blocks plan assumes them): held to 256 registers
-// per lane (unbounded, the partial-tile code took 256 VGPRs + 64 AGPRs).
-template <bool GB>
-__global__ __launch_bounds__(kGThreads, 2) void gemm_latent_sk_kernel(GemmParams p, SkParams q) {
-  const int tid = int(threadIdx.x);
-  const int grp = int(blockIdx.x) % q.G;
-  const int b = int(blockIdx.x) / q.G;
-  const int gb0 = grp * q.P;  // the group's first slot and counter
-  const int64_t it1 = sk_start(b + 1, q);
-  __shared__ int s_last;
-  for (int64_t it = sk_start(b, q); it < it1;) {
-    const int t = int(it / q.nks);
-    const int k0 = int(it - int64_t(t) * q.nks);
-    const int n = int(min<int64_t>(q.nks - k0, it1 - it));
-    const int nt = t % q.NT;
-    const GemmSeg& G = p.seg[latent_segment(p, nt)];
-    const int m0 = ((t / q.NT) * q.G + grp) * kGB;
-    const int c0 = (nt - G.nt0) * kGB;
-    f32x16 acc[kGMI][kGNJ];
-#pragma unroll
-    for (int i = 0; i < kGMI; ++i)
-#pragma unroll
-      for (int j = 0; j < kGNJ; ++j) acc[i][j] = f32x16{};
-    gemm_mainloop<GB>(p.a + G.abase, p.Kp, p.M, m0, G.V, p.KW, G.R, c0, n, acc, tid, G.g, k0);
-    bool store = true;
-    if (n < q.nks) {
-      const int64_t ts = int64_t(t) * q.nks;
-      const int bf = sk_block(ts, q);
-      float* __restrict__ mine = q.part + (size_t(gb0 + b) * 2 + (k0 > 0 ? 0 : 1)) * (64 * kGThreads);
-#pragma unroll
-      for (int i = 0; i < kGMI; ++i)
-#pragma unroll
-        for (int j = 0; j < kGNJ; ++j)
-#pragma unroll
-          for (int e = 0; e < 16; ++e)
-            __hip_atomic_store(mine + ((i * kGNJ + j) * 16 + e) * kGThreads + tid, acc[i][j][e], __ATOMIC_RELAXED,
-                               __HIP_MEMORY_SCOPE_AGENT);
-      __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(0));
-      __syncthreads();
-      if (tid == 0) {
-        const uint32_t before = __hip_atomic_fetch_add(q.cnt + gb0 + bf, uint32_t(n), __ATOMIC_RELAXED,
-                                                       __HIP_MEMORY_SCOPE_AGENT);
-        s_last = before + uint32_t(n) == uint32_t(q.nks) ? 1 : 0;
-      }
-      __syncthreads();
-      store = s_last != 0;
-      if (store) {
-        // the stored parts (this block's too) in block order, whichever
-        // block completes the tile: the sum is the same on every run
-        const int bl = sk_block(ts + q.nks - 1, q);
-#pragma unroll
-        for (int i = 0; i < kGMI; ++i)
-#pragma unroll
-          for (int j = 0; j < kGNJ; ++j) acc[i][j] = f32x16{};
-        for (int o = bf; o <= bl; ++o) {
-          float* __restrict__ part =
-              q.part + (size_t(gb0 + o) * 2 + (sk_start(o, q) > ts ? 0 : 1)) * (64 * kGThreads);
-#pragma unroll
-          for (int i = 0; i < kGMI; ++i)
-#pragma unroll
-            for (int j = 0; j < kGNJ; ++j)
-#pragma unroll
-              for (int e = 0; e < 16; ++e)
-                acc[i][j][e] += __hip_atomic_load(part + ((i * kGNJ + j) * 16 + e) * kGThreads + tid, __ATOMIC_RELAXED,
-                                                  __HIP_MEMORY_SCOPE_AGENT);
-        }
-        if (tid == 0) __hip_atomic_store(q.cnt + gb0 + bf, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      }
-    }
-    if (store) latent_store(p, G, m0, c0, acc, tid);
-    it += n;
-  }
-}
-
-// Stage 2.  grid = (m-tiles, column tiles of all projections), 256 threads.
-// Held to 256 registers per lane (two waves per SIMD; unbounded, the two
-// accumulator sets took 244 VGPRs + 64 AGPRs, one wave per SIMD).
-template <typename YT>
-__global__ __launch_bounds__(kGThreads, 2) void gemm_expand_kernel(GemmParams p) {
-  const int tid = int(threadIdx.x);
-  const int nt = int(blockIdx.y);
-  int pi = 0;
-#pragma unroll
-  for (int i = 1; i < kMaxProj; ++i) pi += (i < p.nproj && nt >= p.proj[i].nt0) ? 1 : 0;
-  pi = __builtin_amdgcn_readfirstlane(pi);
-  const GemmProj& P = p.proj[pi];
-  const int m0 = int(blockIdx.x) * kGB;
-  const int c0 = (nt - P.nt0) * kGB;
-  f32x16 acc0[kGMI][kGNJ], acc1[kGMI][kGNJ];
-#pragma unroll
-  for (int i = 0; i < kGMI; ++i)
-#pragma unroll
-    for (int j = 0; j < kGNJ; ++j) acc0[i][j] = acc1[i][j] = f32x16{};
-  // T rows are zero from R to RP >= 64 * ceil(RW / 2), so whole 64-k steps are safe
-  gemm_mainloop<>(p.t + P.tbase[0], P.RP[0], p.M, m0, P.U[0], P.RW[0], P.N, c0, (P.RW[0] + 1) / 2,
-                       acc0, tid);
-  if (P.nb > 1)
-    gemm_mainloop<>(p.t + P.tbase[1], P.RP[1], p.M, m0, P.U[1], P.RW[1], P.N, c0,
-                         (P.RW[1] + 1) / 2, acc1, tid);
-
-  const int lane = tid & 63, wave = tid >> 6;
-  const int wm = gemm_wm(wave), wn = gemm_wn(wave);
-  const int lr = lane & 31, lh = lane >> 5;
-  YT* __restrict__ y = static_cast<YT*>(P.y);
-#pragma unroll
-  for (int j = 0; j < kGNJ; ++j) {
-    const int n = c0 + gemm_col<kGNJ>(wn, j) + lr;
-    if (n >= P.N) continue;
-    const float h0 = P.h[0][n];
-    const float h1 = P.nb > 1 ? P.h[1][n] : 0.f;
-    const float bn = P.bias ? P.bias[n] : 0.f;
-    const float* res = P.res;
-#pragma unroll
-    for (int i = 0; i < kGMI; ++i)
-#pragma unroll
-      for (int q = 0; q < 16; ++q) {
-        const int m = m0 + gemm_row(wm, i) + 8 * (q >> 2) + 4 * lh + (q & 3);
-        if (m < p.M) {
-          const size_t o = size_t(m) * P.N + n;
-          store_out(y, o, h0 * acc0[i][j][q] + h1 * acc1[i][j][q] + bn + (res ? res[o] : 0.f));
-        }
-      }
-  }
-}
-
-// Stage 2 on bf16 activations in wide tiles.  grid = (m-tiles, 256-column
-// tiles of all projections), 256 threads (4 waves as in gemm_mainloop), one set of
-// accumulators for both branches (two sets would not fit two blocks per CU):
-// acc = S0 after branch 0 (S_b = sum_r sU_b[n, r] * T_b[m, r]), each column's
-// acc times h0 / h1 in fp32, then branch 1 added: y = h1 * acc = h0 * S0 + h1
-// * S1, + bias (+ residual).  Where branch 1 is dropped (use_branch1: h1
-// zero, denormal or below 2^-40 |h0|, where h0 / h1 could overflow acc)
-// branch 1's B operand is 0 and y = h0 * S0; the term dropped is at most
-// 2^-40 of h0 times |S1 / S0|.
-template <typename YT>
-__global__ __launch_bounds__(kGThreads, 2) void gemm_expand_wide_kernel(GemmParams p) {
-  constexpr int BN = 2 * kGB, NJ = gemm_nj<BN>();
-  const int tid = int(threadIdx.x);
-  const int nt = int(blockIdx.y);
-  int pi = 0;
-#pragma unroll
-  for (int i = 1; i < kMaxProj; ++i) pi += (i < p.nproj && nt >= p.proj[i].nt0) ? 1 : 0;
-  pi = __builtin_amdgcn_readfirstlane(pi);
-  const GemmProj& P = p.proj[pi];
-  const int m0 = int(blockIdx.x) * kGB;
-  const int c0 = (nt - P.nt0) * BN;
-  const int lane = tid & 63, wave = tid >> 6;
-  const int wm = gemm_wm(wave), wn = gemm_wn(wave);
-  const int lr = lane & 31, lh = lane >> 5;
-  f32x16 acc[kGMI][NJ];
-#pragma unroll
-  for (int i = 0; i < kGMI; ++i)
-#pragma unroll
-    for (int j = 0; j < NJ; ++j) acc[i][j] = f32x16{};
-  // T rows are zero from R to RP >= 64 * ceil(RW / 2), so whole 64-k steps are safe
-  gemm_mainloop<false, BN>(p.t + P.tbase[0], P.RP[0], p.M, m0, P.U[0], P.RW[0], P.N, c0,
-                                  (P.RW[0] + 1) / 2, acc, tid, nullptr, 0, nullptr);
-  float f[NJ];  // the factor y takes of acc, per subtile column
-#pragma unroll
-  for (int j = 0; j < NJ; ++j) {
-    const int n = min(c0 + gemm_col<NJ>(wn, j) + lr, P.N - 1);
-    const float h0 = P.h[0][n];
-    const float h1 = P.nb > 1 ? P.h[1][n] : 0.f;
-    const bool use1 = P.nb > 1 && use_branch1(h0, h1);
-    f[j] = use1 ? h1 : h0;
-    if (use1) {
-      const float r = h0 / h1;
-#pragma unroll
-      for (int i = 0; i < kGMI; ++i) acc[i][j] *= r;
-    }
-  }
-  if (P.nb > 1)
-    gemm_mainloop<false, BN>(p.t + P.tbase[1], P.RP[1], p.M, m0, P.U[1], P.RW[1], P.N, c0,
-                                    (P.RW[1] + 1) / 2, acc, tid, nullptr, 0, P.h[1], P.h[0]);
-
-  YT* __restrict__ y = static_cast<YT*>(P.y);
-#pragma unroll
-  for (int j = 0; j < NJ; ++j) {
-    const int n = c0 + gemm_col<NJ>(wn, j) + lr;
-    if (n >= P.N) continue;
-    const float bn = P.bias ? P.bias[n] : 0.f;
-    const float* res = P.res;
-#pragma unroll
-    for (int i = 0; i < kGMI; ++i)
-#pragma unroll
-      for (int q = 0; q < 16; ++q) {
-        const int m = m0 + gemm_row(wm, i) + 8 * (q >> 2) + 4 * lh + (q & 3);
-        if (m < p.M) {
-          const size_t o = size_t(m) * P.N + n;
-          store_out(y, o, f[j] * acc[i][j][q] + bn + (res ? res[o] : 0.f));
-        }
-      }
-  }
-}
 
 // hi = bf16(v), lo = bf16(v - hi), round to nearest even
 __device__ __forceinline__ void split1(float v, uint16_t& hi, uint16_t& lo) {
@@ -2601,7 +1942,7 @@ __device__ __forceinline__ void split1(float v, uint16_t& hi, uint16_t& lo) {
   lo = f32_to_bf16(v - bf16_to_f32(hi));
 }
 
-#include "split_gemm.h"
+#include "sign_gemm.h"
 
 // ---------------------------------------------------------------------------
 // Sign pack / unpack (bit-exact with the reference packer)
@@ -3493,66 +2834,23 @@ int validate_group(const ProjDesc* pd, int np, int64_t M, int64_t K) {
 // Workspace layout (byte offsets), fixed so that calls of any shape on one
 // workspace keep its invariants:
 //   [0, 16)                            latent-buffer state (see MfmaParams)
-//   [kSkCntOffset, + 4 kSkMaxBlocks)   stream-K step counters (zero between calls)
 //   [kDetCntOffset, + 4 kDetMaxBlocks) deterministic mode's row-block counters (zero
 //                                      between calls)
 //   [kTOffset, kTOffset + kTBytes)     MFMA-path latent halves
 //   [kChainOffset, + kChainBytes)      chains' latent regions (zero between
 //                                      chains but for the last region)
 //   [kGemmOffset, ...)                 one call's own scratch: GEMM-path A and
-//                                      T planes, then the stream-K partial
-//                                      tiles (kSkPartBytes); or deterministic
-//                                      mode's partial sums
+//                                      T planes, then stage 1's parts; or
+//                                      deterministic mode's partial sums
 constexpr size_t kTOffset = 4096;
 constexpr size_t kTBytes = 2 * size_t(kTHalf) * sizeof(float);
 constexpr size_t kChainOffset = kTOffset + kTBytes;
 constexpr size_t kChainBytes = size_t(kMaxChainLinks) * kChainRegion * sizeof(float);
 constexpr size_t kGemmOffset = kChainOffset + kChainBytes;
 static_assert(kCounterBytes <= kTOffset, "counter region overlaps t");
-constexpr int kNumCUs = 256;                   // MI355X
-constexpr int kSkMaxBlocks = 2 * kNumCUs;      // stream-K blocks: two resident per CU (bf16 stage ring)
-constexpr size_t kSkCntOffset = 256;
-static_assert(kSkCntOffset + kSkMaxBlocks * sizeof(uint32_t) <= kCounterBytes, "stream-K counters");
 constexpr int kDetMaxBlocks = int(kMaxRankTotal / kRowBlock) + kMaxSeg;  // row-blocks of one decode-path call
-constexpr size_t kDetCntOffset = kSkCntOffset + kSkMaxBlocks * sizeof(uint32_t);
+constexpr size_t kDetCntOffset = 2304;
 static_assert(kDetCntOffset + kDetMaxBlocks * sizeof(uint32_t) <= kCounterBytes, "deterministic-mode counters");
-constexpr size_t kSkSlotBytes = size_t(64) * kGThreads * sizeof(float);  // one fp32 partial tile
-
-// Stream-K blocks of stage 1, or 0 when whole tiles do as well.  Costs in
-// k-steps of one block alone on a CU, as measured on the config-4 shapes at
-// M = 128 .. 2048: two co-resident blocks each take 1.5x as long per step,
-// and a stream-K block pays about 24 steps more (its extra ring prologues
-// and the partial tiles).  Whole tiles: nks when each CU gets at most one,
-// else ceil(tiles / 2 CUs) rounds of 1.5 nks.  P stream-K blocks: W / P + 24,
-// times 1.5 when P > CUs.  P is at most the resident slots, about 4 steps
-// per block and 4 parts per tile (the part that completes a tile reads the
-// others' 64 KB partial tiles on its own); the better of P <= CUs and P <=
-// slots, and only if it saves 5 %.
-int64_t sk_blocks(int64_t tiles, int64_t nks, int slots) {
-  if (tiles < 1 || nks < 1) return 0;  // M = 0: nothing to share
-  const int64_t work = tiles * nks, cap = std::min<int64_t>(std::max<int64_t>(1, work / 4), 4 * tiles);
-  // costs doubled, to keep the factor 1.5 in integers
-  const int64_t dp = tiles <= kNumCUs ? 2 * nks : ceil_div(tiles, int64_t(2 * kNumCUs)) * 3 * nks;
-  int64_t best = 0, best_cost = dp * 95 / 100;
-  for (int64_t lim : {int64_t(kNumCUs), int64_t(slots)}) {
-    const int64_t P = std::min(lim, cap);
-    const int64_t cost = (P > kNumCUs ? 3 : 2) * (ceil_div(work, P) + 24);
-    if (cost < best_cost) {
-      best = P;
-      best_cost = cost;
-    }
-  }
-  return best;
-}
-
-// Column tiles of stage 1 over all branches.
-int64_t latent_col_tiles(const ProjDesc* pd, int np) {
-  int64_t nt = 0;
-  for (int q = 0; q < np; ++q)
-    for (int b = 0; b < pd[q].nb; ++b) nt += ceil_div(pd[q].br[b].rank, kGB);
-  return nt;
-}
-
 // Deterministic mode (lbk_set_deterministic): process-wide; read when a
 // call is planned, so a workspace sized while it was off may be too small
 // for a call made after it is turned on (that call returns
@@ -3588,7 +2886,7 @@ struct Plan {
   size_t lds1, lds2;
   bool split;    // seq: the rows run on the split GEMM path where the workspace holds it
   size_t ws_total;  // workspace the fastest form of the call uses
-  size_t ws_min;    // workspace it needs (GEMM path: without the stream-K partial tiles)
+  size_t ws_min;    // workspace it needs (GEMM path: without stage 1's parts)
 };
 
 int mtile(int64_t M) { return M <= 1 ? 1 : M <= 2 ? 2 : M <= 4 ? 4 : M <= 8 ? 8 : 16; }
@@ -3600,44 +2898,44 @@ size_t compact_rows(int mt, int64_t nch) {
 }
 
 
-// Elements per plane of the GEMM path's A (per segment [M][Kp]) and T (per
-// segment [M][RP]); planes are bf16, two of each (hi, lo) for fp32 activations.
-void gemm_planes(const ProjDesc* pd, int np, int64_t M, int64_t K, int64_t& a_plane, int64_t& t_plane) {
-  a_plane = t_plane = 0;
-  const int64_t Kp = ceil_div(K, kGK) * kGK;
+// Bytes of the GEMM path's A (per segment [M][K rounded up to 64]) and T (per
+// segment [M][R rounded up to 128]) in `planes` bf16 planes (fp32 activations:
+// hi and lo).
+size_t gemm_ws_bytes(const ProjDesc* pd, int np, int64_t M, int64_t K, int planes) {
+  int64_t ap = 0, tp = 0;
   for (int q = 0; q < np; ++q)
     for (int b = 0; b < pd[q].nb; ++b) {
-      a_plane += M * Kp;
-      t_plane += M * ceil_div(pd[q].br[b].rank, kGB) * kGB;
+      ap += M * ceil_div(K, 64) * 64;
+      tp += M * ceil_div(pd[q].br[b].rank, 128) * 128;
     }
+  return align256(size_t(ap) * planes * sizeof(uint16_t)) + align256(size_t(tp) * planes * sizeof(uint16_t));
 }
 
-// Room for two planes of each (a query does not know the activations' type).
-size_t gemm_ws_bytes(const ProjDesc* pd, int np, int64_t M, int64_t K) {
-  int64_t ap, tp;
-  gemm_planes(pd, np, M, K, ap, tp);
-  return align256(size_t(ap) * 2 * sizeof(uint16_t)) + align256(size_t(tp) * 2 * sizeof(uint16_t));
-}
-
-// Launch shape of the split GEMM path (split_gemm.h), from a sweep of every
-// (rows, columns, parts) over single and grouped Llama-2 / Llama-3 calls, one
-// and two branches, M = 33 .. 2048; the choices are within about 5 % of the
-// best shape of each stage.  Tiles are counted as 32 x 128.
+// Launch shape of the GEMM path (sign_gemm.h), from sweeps of every (rows,
+// columns, parts) over single and grouped Llama-2 / Llama-3 calls, one and two
+// branches, M = 33 .. 2048, fp32 (split) and bf16 activations; the choices are
+// within about 5 % of the best shape of each stage.  Tiles are counted as 32 x
+// 128.
 //   Stage 1: 32 x 128 tiles, the k range in parts while there are fewer than
-//   about 512 blocks (two per CU): M = 300, one 4096 -> 4096 projection of
-//   ranks 205 + 1843, 170 tiles, 24.5 us whole and 22.2 us in 3 parts; M =
-//   2048, gate and up, 3072 tiles, 178.6 us against 167.3 us in 64-row tiles.
-//   Stage 2: 32 x 128 tiles while they are few (M = 512, 4096 columns: 512
-//   tiles 22.2 us, 64 x 128 27.1 us, 64 x 256 43.8 us) or the ranks are short
-//   (each tile then mostly stores y), 64 x 256 where those give 600 blocks (M
-//   = 1024, gate and up: 217.6 us against 227.4 us as 64 x 128 and 251.5 us
-//   as 32 x 128), else 64 x 128.
+//   about 512 blocks (two per CU): fp32, M = 300, one 4096 -> 4096 projection
+//   of ranks 205 + 1843, 170 tiles, 24.5 us whole and 22.2 us in 3 parts.
+//   64-row tiles (fewer expansions and words per MFMA) past 1,500 tiles (fp32,
+//   M = 2048, gate and up, 3072 tiles: 178.6 -> 167.3 us) or 700 (bf16, one
+//   MFMA per product: M = 1024, gate and up, 1536 tiles 72.8 -> 60.1 us; 544
+//   tiles 37.4 us against 41.1 us), and over long rows, in parts for three
+//   blocks per CU (bf16, M = 1024, 11008 -> 4096: 86.2 us against 96.5 us in
+//   768 tiles of 32 rows and 100.1 us in 384 whole tiles of 64).
+//   Stage 2: 32 x 128 tiles while they are few (fp32, M = 512, 4096 columns:
+//   512 tiles 22.2 us, 64 x 128 27.1 us, 64 x 256 43.8 us) or the ranks are
+//   short (each tile then mostly stores y), 64 x 256 where those give 600
+//   blocks (fp32, M = 1024, gate and up: 217.6 us against 227.4 us as 64 x 128
+//   and 251.5 us as 32 x 128; bf16 141.3, 146.0, 174.6 us), else 64 x 128.
 struct SgPlan {
   int mi1, parts;  // stage 1: 32 mi1 rows x 128 columns, parts of the k range
   int mi2, nj2;    // stage 2: 32 mi2 rows x 128 nj2 columns
   size_t part_bytes;
 };
-SgPlan sg_plan(const ProjDesc* pd, int np, int64_t M, int64_t K) {
+SgPlan sg_plan(const ProjDesc* pd, int np, int64_t M, int64_t K, bool split) {
   int64_t c1 = 0, cols = 0, c2 = 0, c2w = 0, steps = 0;
   for (int q = 0; q < np; ++q) {
     int64_t st = 0;
@@ -3652,16 +2950,23 @@ SgPlan sg_plan(const ProjDesc* pd, int np, int64_t M, int64_t K) {
   }
   cols = 128 * c1;
   SgPlan s{};
-  const int64_t tiles1 = std::max<int64_t>(1, ceil_div(M, 32)) * c1;  // M = 0: a query
-  s.mi1 = tiles1 < 1500 ? 1 : 2;
-  s.parts = 1;
-  if (s.mi1 == 1) {
-    const int64_t groups = ceil_div(K, 128);  // at least two groups of steps per part
-    s.parts = int(std::max<int64_t>(1, std::min<int64_t>({(512 + tiles1 / 2) / tiles1, 8, groups / 2})));
+  const int64_t rows1 = std::max<int64_t>(1, ceil_div(M, 32));  // M = 0: a query
+  const int64_t tiles1 = rows1 * c1, tiles2 = (rows1 + 1) / 2 * c1;
+  s.mi1 = s.parts = 1;
+  int64_t parts = 1;
+  if (K >= 8192 && tiles2 >= 96) {
+    s.mi1 = 2;
+    parts = (768 + tiles2 / 2) / tiles2;
+  } else if (tiles1 > (split ? 1500 : 700)) {
+    s.mi1 = 2;
+  } else {
+    parts = (512 + tiles1 / 2) / tiles1;
   }
+  // at least two groups of words per part
+  s.parts = int(std::max<int64_t>(1, std::min<int64_t>({parts, 8, ceil_div(K, 128) / 2})));
   s.part_bytes = s.parts > 1 ? size_t(s.parts) * size_t(M) * size_t(cols) * sizeof(float) : 0;
   s.mi2 = s.nj2 = 1;
-  if (ceil_div(M, 32) * c2 > 1100 && steps > 16) {
+  if (ceil_div(M, 32) * c2 > (split ? 1100 : 800) && steps > 16) {
     s.mi2 = 2;
     s.nj2 = ceil_div(M, 64) * c2w >= 600 ? 2 : 1;
   }
@@ -3870,10 +3175,8 @@ Plan plan_one(const ProjDesc* pd, int np, int64_t M, int64_t K, bool allow_ks, b
     if (det && pl.nkc > 1)
       pl.ws_total = pl.ws_min = kGemmOffset + align256(det_part_floats(pd, np, M, pl.nkc) * sizeof(float));
   } else {
-    pl.ws_min = kGemmOffset + gemm_ws_bytes(pd, np, M, K);
-    const int64_t tiles = ceil_div(M, kGB) * latent_col_tiles(pd, np), nks = ceil_div(K, kGK);
-    const int64_t P = sk_blocks(tiles, nks, 2 * kNumCUs);
-    pl.ws_total = pl.ws_min + std::max(size_t(2 * P) * kSkSlotBytes, sg_plan(pd, np, M, K).part_bytes);
+    pl.ws_min = kGemmOffset + gemm_ws_bytes(pd, np, M, K, 2);
+    pl.ws_total = pl.ws_min + std::max(sg_plan(pd, np, M, K, true).part_bytes, sg_plan(pd, np, M, K, false).part_bytes);
   }
   return pl;
 }
@@ -4132,33 +3435,47 @@ int forward_mfma(const ProjDesc* pd, int np, const Plan& pl, int64_t M, int64_t 
   return check_launch("expand_mfma_kernel");
 }
 
-template <typename YT>
+template <typename YT, bool SPLIT>
 void launch_sg_expand(const SgParams& p, const SgPlan& sp, dim3 grid, hipStream_t s) {
-  if (sp.nj2 == 2) hipLaunchKernelGGL((sg_expand_kernel<YT, 2, 2>), grid, dim3(kBlock), 0, s, p);
-  else if (sp.mi2 == 2) hipLaunchKernelGGL((sg_expand_kernel<YT, 2, 1>), grid, dim3(kBlock), 0, s, p);
-  else hipLaunchKernelGGL((sg_expand_kernel<YT, 1, 1>), grid, dim3(kBlock), 0, s, p);
+  if (sp.nj2 == 2) hipLaunchKernelGGL((sg_expand_kernel<YT, SPLIT, 2, 2>), grid, dim3(kBlock), 0, s, p);
+  else if (sp.mi2 == 2) hipLaunchKernelGGL((sg_expand_kernel<YT, SPLIT, 2, 1>), grid, dim3(kBlock), 0, s, p);
+  else hipLaunchKernelGGL((sg_expand_kernel<YT, SPLIT, 1, 1>), grid, dim3(kBlock), 0, s, p);
+}
+template <bool SPLIT, bool GB>
+void launch_sg_latent(const SgParams& p, const SgPlan& sp, dim3 grid, hipStream_t s) {
+  if (sp.mi1 == 2) hipLaunchKernelGGL((sg_latent_kernel<SPLIT, GB, 2>), grid, dim3(kBlock), 0, s, p);
+  else hipLaunchKernelGGL((sg_latent_kernel<SPLIT, GB, 1>), grid, dim3(kBlock), 0, s, p);
 }
 
-// Workspace of a split-GEMM call: A and T, then stage 1's parts.
+// Workspace of a split call (fp32 sums of hi and lo planes): A and T, then
+// stage 1's parts.
 size_t sg_ws_bytes(const ProjDesc* pd, int np, int64_t M, int64_t K) {
-  return kGemmOffset + gemm_ws_bytes(pd, np, M, K) + sg_plan(pd, np, M, K).part_bytes;
+  return kGemmOffset + gemm_ws_bytes(pd, np, M, K, 2) + sg_plan(pd, np, M, K, true).part_bytes;
 }
 
-// A call on the split GEMM path (split_gemm.h).  x is read by the first
-// kernel only, so an output may share its memory.  A workspace without room
-// for stage 1's parts runs whole tiles.
-int forward_split(const ProjDesc* pd, int np, int64_t M, int64_t K, const void* x, int x_dtype, const InputDesc& in,
-                  int y_dtype, void* workspace, size_t workspace_bytes, hipStream_t s) {
-  SgPlan sp = sg_plan(pd, np, M, K);
-  const size_t planes = gemm_ws_bytes(pd, np, M, K);
+// A call on the GEMM path (sign_gemm.h).  `split`: hi and lo planes, for fp32
+// activations (and bf16 ones that the decode path would have run in fp32);
+// else one bf16 plane.  x is read by the first kernel only where a scaled
+// copy of it is made; bf16 rows of whole 64-k steps at a 16-byte aligned
+// address are read as they are (`direct`), by stage 1, before any output is
+// written, so an output may share x's memory either way.  A workspace without
+// room for stage 1's parts runs whole tiles.
+int forward_gemm(const ProjDesc* pd, int np, int64_t M, int64_t K, const void* x, int x_dtype, bool split,
+                 const InputDesc& in, int y_dtype, void* workspace, size_t workspace_bytes, hipStream_t s) {
+  SgPlan sp = sg_plan(pd, np, M, K, split);
+  const size_t planes = gemm_ws_bytes(pd, np, M, K, split ? 2 : 1);
+  if (workspace_bytes < kGemmOffset + planes)
+    return set_error(LBK_ERR_WORKSPACE, "workspace of %zu bytes needed, %zu given", kGemmOffset + planes,
+                     workspace_bytes);
   if (sp.parts > 1 && workspace_bytes < kGemmOffset + planes + sp.part_bytes) sp.parts = 1;
+  const bool direct = !split && in.kind == LBK_INPUT_PLAIN && K % 64 == 0 && aligned16(x);
   SgParams p;
   memset(&p, 0, sizeof(p));
   p.nproj = np;
   p.M = int(M);
   p.K = int(K);
   p.KW = int(ceil_div(K, 32));
-  p.lda = 64 * p.KW;
+  p.lda = split ? 64 * p.KW : int(ceil_div(K, 64) * 64);
   p.x = x;
   p.x1 = in.x1;
   p.nw = in.nw;
@@ -4192,7 +3509,7 @@ int forward_split(const ProjDesc* pd, int np, int64_t M, int64_t K, const void* 
       S.RP = 128 * P.ng[b];
       S.tcol = tcol;
       S.nt0 = int(nt1);
-      S.abase = abase;
+      S.abase = direct ? 0 : abase;
       nt1 += P.ng[b];
       tcol += S.RP;
       abase += M * p.lda;
@@ -4200,154 +3517,53 @@ int forward_split(const ProjDesc* pd, int np, int64_t M, int64_t K, const void* 
     }
   }
   p.nseg = si;
-  p.ldt = 2 * tcol;
+  p.tcols = tcol;
+  p.ldt = split ? 2 * tcol : tcol;
   p.xvec = xvec ? 1 : 0;
   char* ws = static_cast<char*>(workspace) + kGemmOffset;
-  p.a = reinterpret_cast<uint16_t*>(ws);
+  p.a = direct ? const_cast<uint16_t*>(static_cast<const uint16_t*>(x)) : reinterpret_cast<uint16_t*>(ws);
   p.t = reinterpret_cast<uint16_t*>(ws + align256(size_t(abase) * sizeof(uint16_t)));
   p.part = reinterpret_cast<float*>(ws + planes);
   const int64_t blocks1 = ceil_div(M, 32 * sp.mi1) * nt1 * sp.parts, blocks2 = ceil_div(M, 32 * sp.mi2) * nt2;
-  if (nt1 > 65535 || ceil_div(nt2, 2) > 65535 || blocks1 > INT_MAX || blocks2 > INT_MAX)
+  int64_t nt128 = 0;
+  for (int q = 0; q < np; ++q) nt128 += ceil_div(pd[q].N, 128);
+  if (nt1 > 65535 || nt128 > 65535 || blocks1 > INT_MAX || blocks2 > INT_MAX)
     return set_error(LBK_ERR_ARG, "too many column tiles for the GEMM path");
 
-  const dim3 g0(unsigned(M), unsigned(ceil_div(p.KW, 64)));
-  if (x_dtype == LBK_F32) hipLaunchKernelGGL(sg_scale_kernel<float>, g0, dim3(kBlock), 0, s, p);
-  else hipLaunchKernelGGL(sg_scale_kernel<uint16_t>, g0, dim3(kBlock), 0, s, p);
-  int rc = check_launch("sg_scale_kernel");
-  if (rc != LBK_OK) return rc;
+  int rc;
+  if (!direct) {
+    const dim3 g0(unsigned(M), unsigned(ceil_div(p.lda, (split ? 16 : 8) * kBlock)));
+    if (!split) hipLaunchKernelGGL((sg_scale_kernel<uint16_t, false>), g0, dim3(kBlock), 0, s, p);
+    else if (x_dtype == LBK_F32) hipLaunchKernelGGL((sg_scale_kernel<float, true>), g0, dim3(kBlock), 0, s, p);
+    else hipLaunchKernelGGL((sg_scale_kernel<uint16_t, true>), g0, dim3(kBlock), 0, s, p);
+    rc = check_launch("sg_scale_kernel");
+    if (rc != LBK_OK) return rc;
+  }
   p.parts = sp.parts;
   p.NT = int(nt1);
   const dim3 g1{unsigned(blocks1), 1u, 1u}, g2{unsigned(blocks2), 1u, 1u};
-  if (sp.mi1 == 1) hipLaunchKernelGGL(sg_latent_kernel<1>, g1, dim3(kBlock), 0, s, p);
-  else hipLaunchKernelGGL(sg_latent_kernel<2>, g1, dim3(kBlock), 0, s, p);
+  if (split) launch_sg_latent<true, false>(p, sp, g1, s);
+  else if (direct) launch_sg_latent<false, true>(p, sp, g1, s);
+  else launch_sg_latent<false, false>(p, sp, g1, s);
   rc = check_launch("sg_latent_kernel");
   if (rc != LBK_OK) return rc;
   if (sp.parts > 1) {
     const dim3 gr(unsigned(ceil_div(M * tcol, 4 * kBlock)));
-    hipLaunchKernelGGL(sg_reduce_t_kernel, gr, dim3(kBlock), 0, s, p);
+    if (split) hipLaunchKernelGGL(sg_reduce_t_kernel<true>, gr, dim3(kBlock), 0, s, p);
+    else hipLaunchKernelGGL(sg_reduce_t_kernel<false>, gr, dim3(kBlock), 0, s, p);
     rc = check_launch("sg_reduce_t_kernel");
     if (rc != LBK_OK) return rc;
   }
   p.parts = 1;
   p.NT = int(nt2);
-  if (y_dtype == LBK_F32) launch_sg_expand<float>(p, sp, g2, s);
-  else launch_sg_expand<uint16_t>(p, sp, g2, s);
-  return check_launch("sg_expand_kernel");
-}
-
-int forward_gemm(const ProjDesc* pd, int np, int64_t M, int64_t K, const void* x, int x_dtype, const InputDesc& in,
-                 int y_dtype, void* workspace, size_t workspace_bytes, hipStream_t s) {
-  if (x_dtype == LBK_F32) return forward_split(pd, np, M, K, x, x_dtype, in, y_dtype, workspace, workspace_bytes, s);
-  GemmParams p;
-  memset(&p, 0, sizeof(p));
-  p.nproj = np;
-  p.M = int(M);
-  p.K = int(K);
-  p.KW = int(ceil_div(K, 32));
-  p.Kp = int(ceil_div(K, kGK) * kGK);
-  p.x = x;
-  int64_t a_plane, t_plane;
-  gemm_planes(pd, np, M, K, a_plane, t_plane);
-  char* ws = static_cast<char*>(workspace) + kGemmOffset;
-  p.a = reinterpret_cast<uint16_t*>(ws);
-  p.t = reinterpret_cast<uint16_t*>(ws + align256(size_t(a_plane) * sizeof(uint16_t)));
-  p.xmode = in.kind;
-  p.x1 = in.x1;
-  p.nw = in.nw;
-  p.eps = in.eps;
-  bool xvec = (K % 8) == 0 && aligned16(x) && (!in.x1 || aligned16(in.x1)) && (!in.nw || aligned16(in.nw));
-  int si = 0, nt1 = 0, nt2 = 0;
-  int64_t abase = 0, tbase = 0;
-  for (int q = 0; q < np; ++q) {
-    GemmProj& P = p.proj[q];
-    P.nb = pd[q].nb;
-    P.N = int(pd[q].N);
-    P.bias = pd[q].bias;
-    P.res = pd[q].res;
-    P.y = pd[q].y;
-    P.nt0 = nt2;
-    nt2 += int(ceil_div(pd[q].N, kGB));
-    for (int b = 0; b < pd[q].nb; ++b, ++si) {
-      const lbk_branch& B = pd[q].br[b];
-      GemmSeg& S = p.seg[si];
-      S.V = reinterpret_cast<const uint32_t*>(B.v_sign);
-      S.g = B.v2;
-      S.l = B.mid;
-      S.R = int(B.rank);
-      S.RP = int(ceil_div(B.rank, kGB) * kGB);
-      S.nt0 = nt1;
-      S.abase = abase;
-      S.tbase = tbase;
-      nt1 += S.RP / kGB;
-      abase += M * p.Kp;
-      P.U[b] = reinterpret_cast<const uint32_t*>(B.u_sign);
-      P.h[b] = B.u1;
-      P.RW[b] = int(ceil_div(B.rank, 32));
-      P.RP[b] = S.RP;
-      P.tbase[b] = tbase;
-      tbase += M * S.RP;
-      xvec = xvec && (reinterpret_cast<uintptr_t>(B.v2) % 16) == 0;
-    }
-  }
-  p.nseg = si;
-  p.xvec = xvec ? 1 : 0;
-  const int64_t mtiles = ceil_div(M, kGB);
-  if (nt1 > 65535 || nt2 > 65535) return set_error(LBK_ERR_ARG, "too many column tiles for the GEMM path");
-  const size_t lds = 0;  // the stage ring is static LDS
-  const dim3 g0{unsigned(M), unsigned(si), 1u};
-  const dim3 g1{unsigned(mtiles), unsigned(nt1), 1u}, g2{unsigned(mtiles), unsigned(nt2), 1u};
-  // bf16 rows of whole k-steps, taken as they are: g goes into stage 1's B
-  // operand and no scaled copy of x is made
-  const bool direct = in.kind == LBK_INPUT_PLAIN && K % kGK == 0 && aligned16(x);
-  // Stream-K stage 1 when whole tiles would leave the block slots unevenly
-  // used (estimated in k-steps of one block: rounds of tiles vs an even
-  // share plus about two steps for the partial tiles), and the workspace
-  // holds the partial tiles.
-  const int64_t nks = p.Kp / kGK, tiles = mtiles * nt1;
-  const size_t part_off = kGemmOffset + gemm_ws_bytes(pd, np, M, K);
-  const int64_t P = sk_blocks(tiles, nks, 2 * kNumCUs);  // blocks resident at once (LDS of the stage ring)
-  const bool sk = P > 0 && workspace_bytes >= part_off + size_t(2 * P) * kSkSlotBytes;
-  SkParams q{};
-  q.G = mtiles % 8 == 0 && P % 8 == 0 ? 8 : 1;
-  q.P = int(std::max<int64_t>(P, 1)) / q.G;
-  q.NT = nt1;
-  q.nks = int(nks);
-  q.W = tiles / q.G * nks;
-  q.part = reinterpret_cast<float*>(static_cast<char*>(workspace) + part_off);
-  q.cnt = reinterpret_cast<uint32_t*>(static_cast<char*>(workspace) + kSkCntOffset);
-  const dim3 gsk{unsigned(q.G * q.P), 1u, 1u};
-  int rc;
-  if (direct) {
-    p.a = const_cast<uint16_t*>(static_cast<const uint16_t*>(x));
-    for (int i = 0; i < si; ++i) p.seg[i].abase = 0;
-    if (sk) hipLaunchKernelGGL(gemm_latent_sk_kernel<true>, gsk, dim3(kGThreads), 0, s, p, q);
-    else hipLaunchKernelGGL(gemm_latent_kernel<true>, g1, dim3(kGThreads), lds, s, p);
+  if (split) {
+    if (y_dtype == LBK_F32) launch_sg_expand<float, true>(p, sp, g2, s);
+    else launch_sg_expand<uint16_t, true>(p, sp, g2, s);
   } else {
-    hipLaunchKernelGGL(gemm_scale_kernel<uint16_t>, g0, dim3(kGThreads), 0, s, p);
-    rc = check_launch("gemm_scale_kernel");
-    if (rc != LBK_OK) return rc;
-    if (sk) hipLaunchKernelGGL(gemm_latent_sk_kernel<false>, gsk, dim3(kGThreads), 0, s, p, q);
-    else hipLaunchKernelGGL(gemm_latent_kernel<false>, g1, dim3(kGThreads), lds, s, p);
+    if (y_dtype == LBK_F32) launch_sg_expand<float, false>(p, sp, g2, s);
+    else launch_sg_expand<uint16_t, false>(p, sp, g2, s);
   }
-  rc = check_launch("gemm_latent_kernel");
-  if (rc != LBK_OK) return rc;
-  // 256-column tiles where they still give every CU two
-  // blocks (the stage ring allows two per CU); else 128-column tiles
-  int ntw = 0;
-  for (int q = 0; q < np; ++q) ntw += int(ceil_div(pd[q].N, 2 * kGB));
-  if (mtiles * ntw >= 2 * kNumCUs && ntw <= 65535) {
-    for (int q = 0, t = 0; q < np; ++q) {
-      p.proj[q].nt0 = t;
-      t += int(ceil_div(pd[q].N, 2 * kGB));
-    }
-    const dim3 gw{unsigned(mtiles), unsigned(ntw), 1u};
-    if (y_dtype == LBK_F32) hipLaunchKernelGGL((gemm_expand_wide_kernel<float>), gw, dim3(kGThreads), lds, s, p);
-    else hipLaunchKernelGGL((gemm_expand_wide_kernel<uint16_t>), gw, dim3(kGThreads), lds, s, p);
-    return check_launch("gemm_expand_wide_kernel");
-  }
-  if (y_dtype == LBK_F32) hipLaunchKernelGGL((gemm_expand_kernel<float>), g2, dim3(kGThreads), lds, s, p);
-  else hipLaunchKernelGGL((gemm_expand_kernel<uint16_t>), g2, dim3(kGThreads), lds, s, p);
-  return check_launch("gemm_expand_kernel");
+  return check_launch("sg_expand_kernel");
 }
 
 bool overlaps(const void* a, size_t na, const void* b, size_t nb) {
@@ -4491,7 +3707,9 @@ int run_group(const ProjDesc* pd, int np, int64_t M, int64_t K, const void* x, i
               int y_dtype, const Plan& pl, void* workspace, size_t workspace_bytes, void* stream) {
   if (M == 0) return LBK_OK;
   int rc = LBK_OK;
-  if (!workspace || workspace_bytes < pl.ws_min)
+  // on the GEMM path a bf16 call needs one plane, not the two that a query
+  // allows for (forward_gemm checks what its call needs)
+  if (!workspace || (workspace_bytes < pl.ws_min && (pl.mfma || x_dtype == LBK_F32)))
     return set_error(LBK_ERR_WORKSPACE, "workspace of %zu bytes needed, %zu given", pl.ws_min, workspace_bytes);
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (pl.chunk > 0 && !pl.seq) {
@@ -4500,7 +3718,7 @@ int run_group(const ProjDesc* pd, int np, int64_t M, int64_t K, const void* x, i
     return forward_mfma(pd, np, pl, M, K, x, x_dtype, in, y_dtype, workspace, s);
   }
   if (pl.split && workspace_bytes >= sg_ws_bytes(pd, np, M, K))
-    return forward_split(pd, np, M, K, x, x_dtype, in, y_dtype, workspace, workspace_bytes, s);
+    return forward_gemm(pd, np, M, K, x, x_dtype, true, in, y_dtype, workspace, workspace_bytes, s);
   if (pl.chunk > 0) {
     // one launch pair per chunk (deterministic mode sizes its partials for
     // one chunk; or the rows' t does not fit the latent half at once)
@@ -4528,7 +3746,7 @@ int run_group(const ProjDesc* pd, int np, int64_t M, int64_t K, const void* x, i
     return LBK_OK;
   }
   if (pl.mfma) return forward_mfma(pd, np, pl, M, K, x, x_dtype, in, y_dtype, workspace, s);
-  return forward_gemm(pd, np, M, K, x, x_dtype, in, y_dtype, workspace, workspace_bytes, s);
+  return forward_gemm(pd, np, M, K, x, x_dtype, x_dtype == LBK_F32, in, y_dtype, workspace, workspace_bytes, s);
 }
 
 int forward_group(const ProjDesc* pd, int np, int64_t M, int64_t K, const void* x, int x_dtype,

@@ -1,32 +1,39 @@
-// Split GEMM path: fp32 activations, more rows than the decode path takes at
-// its best.  Included by littlebit_amd.hip inside its anonymous namespace.
+// GEMM path: more rows than the decode path takes.  Included by
+// littlebit_amd.hip inside its anonymous namespace.
 //
-//   sg_scale_kernel   A_s[m, k] = g_s[k] * input[m, k] per branch s, as bf16
-//                     hi and lo = bf16(v - hi)
-//   sg_latent_kernel  T_s[m, r] = l_s[r] * sum_k sV_s[r, k] * A_s[m, k], as hi / lo
+//   sg_scale_kernel   A_s[m, k] = g_s[k] * input[m, k] per branch s, where the
+//                     input cannot be read as it is
+//   sg_latent_kernel  T_s[m, r] = l_s[r] * sum_k sV_s[r, k] * A_s[m, k]
+//   sg_reduce_t_kernel  T from the fp32 tiles of the parts, in part order, where
+//                     stage 1's k range is cut into parts so that enough blocks
+//                     run side by side (every call repeats bit for bit)
 //   sg_expand_kernel  y[m, n] = bias[n] + sum_b h_b[n] * sum_r sU_b[n, r] * T_b[m, r]
-// and, where the k range of a stage's tiles is cut into parts so that enough
-// blocks run side by side, a kernel that sums the parts' fp32 tiles in part
-// order (sg_reduce_t_kernel, sg_reduce_y_kernel): every call repeats bit for
-// bit.
 //
-// A and T rows interleave the two planes per sign word: 32 hi values then
-// the 32 lo values of the same k, 128 bytes.  One k-step is one sign word per
-// column: a 128-byte row segment holds both planes' operands of it, so a
-// +-1 operand expanded from the word feeds the hi and the lo MFMA, and the
-// stage ring is that of a 64-k step of plain bf16.
+// SPLIT (fp32 activations): A and T as bf16 hi and lo = bf16(v - hi), both
+// through the MFMAs, so products keep ~2^-17 relative error.  Rows interleave
+// the planes per sign word, 32 hi values then the 32 lo values of the same k,
+// 128 bytes.  One k-step is one sign word per column: a 128-byte row segment
+// holds both planes' operands of it, and a +-1 operand expanded from the word
+// feeds the hi and the lo MFMA.  Without (bf16 activations) one plane, the
+// precision of the reference's bf16 forward (littlebit.py:116-121); a 128-byte
+// step is 64 k, two words.  bf16 rows of whole steps are read as they are (GB),
+// with g, rounded to bf16, in the B operand.
 //
-// What bounds it: the MFMAs, two per product.  At M = 1024 gate and up of the
-// Llama-2 target (4096 -> 2 x 11008, ranks 298 + 2686) run 369 GFLOP of them
-// in 328 us, 1.13 PFLOP/s, where an 8192^3 bf16 library product reaches 1.19
-// on the same card; a call of few tiles is bound by its chain of steps (M =
-// 300, 4096 -> 4096, ranks 205 + 1843: 48 us, 0.42 PFLOP/s).  128-row tiles
-// with a 64-k step of two separate planes (128 KB of LDS ring, one wave per
-// SIMD, and two accumulator sets) took 506 us and 94 us; here a block needs
-// 16 KB or 32 KB of LDS and at most 128 registers, so four waves per SIMD
-// hide each other's LDS reads, barriers and expansions.  A stage of four
-// steps per barrier for the 32-row tiles measured no faster (M = 300 stage 2
-// 21.0 -> 23.3 us: three blocks per CU instead of seven).
+// What bounds it: the MFMAs of large calls.  fp32, M = 1024, gate and up of the
+// Llama-2 target (4096 -> 2 x 11008, ranks 298 + 2686): 369 GFLOP (two MFMAs per
+// product) in 328 us, 1.13 PFLOP/s, where an 8192^3 bf16 library product reaches
+// 1.19 on the same card.  bf16, M = 2048, the Llama-3 gate (4096 -> 14336, ranks
+// 318 + 2867): 240 GFLOP in 240 us, 1.00 PFLOP/s (9 VALU per expanded operand
+// and 2 MFMAs).  A call of few tiles is bound by its chain of steps, about 340
+// cycles each without any memory access (fp32, M = 300, 4096 -> 4096, ranks 205
+// + 1843: 48 us, 0.42 PFLOP/s).  128-row tiles with 64 KB (bf16) or 128 KB
+// (fp32, separate planes, two accumulator sets) of LDS ring, two and one waves
+// per SIMD, took 506, 255 and 94 us for the three, and 43 us against 19 for a
+// bf16 draft projection of rank 205 at M = 300; here a block needs 16 or 32 KB
+// of LDS and at most 128 registers, so four waves per SIMD hide each other's LDS
+// reads, barriers and expansions.  A stage of four steps per barrier for the
+// 32-row tiles measured no faster (fp32, M = 300, stage 2: 21.0 -> 23.3 us,
+// three blocks per CU instead of seven).
 
 struct SgSeg {         // stage-1 operands of one branch
   const uint32_t* V;   // [R, KW]
@@ -59,8 +66,9 @@ struct SgParams {
   SgProj proj[kMaxProj];
   int nseg, nproj;
   int M, K, KW;
-  int lda;             // elements per A row, 64 * KW
-  int ldt;             // elements per T row, 2 * sum of RP
+  int lda;             // elements per A row: 64 KW split, else K rounded up to 64 (K of x itself)
+  int ldt;             // elements per T row: tcols, twice that split
+  int tcols;           // latent columns of a row, the sum of RP
   int xvec;            // x (x1, rms weight) rows and every g allow 16-byte loads
   int xmode;           // LBK_INPUT_*
   const void* x;
@@ -69,7 +77,7 @@ struct SgParams {
   float eps;
   uint16_t* a;
   uint16_t* t;
-  float* part;         // stage 1's parts of the k range: [parts][M][ldt / 2] fp32
+  float* part;         // stage 1's parts of the k range: [parts][M][tcols] fp32
   int parts;           // 1: tiles store T themselves
   int NT;              // column tiles over all segments / projections
 };
@@ -80,7 +88,7 @@ struct SgParams {
 // 700, K = 4096 writes 69 MB (a block per row and segment took 32 us; this
 // about 15).
 // grid = (M, ceil(32 KW / (8 * 256))).
-template <typename XT>
+template <typename XT, bool SPLIT>
 __global__ __launch_bounds__(kBlock) void sg_scale_kernel(SgParams p) {
   const int m = int(blockIdx.x), tid = int(threadIdx.x);
   const XT* __restrict__ xr = static_cast<const XT*>(p.x) + int64_t(m) * p.K;
@@ -104,7 +112,7 @@ __global__ __launch_bounds__(kBlock) void sg_scale_kernel(SgParams p) {
     rsm = rs[0];
   }
   const int k = 8 * (int(blockIdx.y) * kBlock + tid);
-  if (k >= 32 * p.KW) return;
+  if (k >= (SPLIT ? 32 * p.KW : p.lda)) return;
   float v[8];
   const bool vec = p.xvec && k + 8 <= p.K;
   if (vec) {
@@ -132,7 +140,7 @@ __global__ __launch_bounds__(kBlock) void sg_scale_kernel(SgParams p) {
       v[i] = e;
     }
   }
-  uint16_t* __restrict__ out = p.a + int64_t(m) * p.lda + (k >> 5) * 64 + (k & 31);
+  uint16_t* __restrict__ out = p.a + int64_t(m) * p.lda + (SPLIT ? (k >> 5) * 64 + (k & 31) : k);
   for (int s = 0; s < p.nseg; ++s) {
     const float* __restrict__ g = p.seg[s].g;
     float a[8];
@@ -148,129 +156,173 @@ __global__ __launch_bounds__(kBlock) void sg_scale_kernel(SgParams p) {
     split8(a, h, l);
     uint16_t* o = out + p.seg[s].abase;
     *reinterpret_cast<u32x4*>(o) = h;
-    *reinterpret_cast<u32x4*>(o + 32) = l;
+    if constexpr (SPLIT) *reinterpret_cast<u32x4*>(o + 32) = l;
   }
 }
 
-// acc[i][j] += A[m0 + 32 i + .., both planes of steps s0 .. s1) . S[.., c + 32 j + ..]
-// A: rows of interleaved 128-byte steps, `src` the lane's DMA sources of step
-// s0; words(g) loads the lane's columns' sign words of steps 4 g .. 4 g + 3
-// (s0 a multiple of 4); boundary(g) runs before group g's MFMAs.
+// acc[i][j] += A[m0 + 32 i + .., steps 0 .. n) . S[.., c + 32 j + ..]
+// A: rows of 128-byte steps, `src` the lane's DMA sources of step 0; words(g)
+// loads the lane's columns' sign words of group g0 + g (4 words: 4 steps of
+// one word with SPLIT, 2 steps of two without); boundary(g) runs before group
+// g's MFMAs.  GB: the B operand is +-g[k] (gk = g of step 0).
 //
 // The block's tile is 32 MI rows x 128 NJ columns, wave w of 4 taking
 // columns 32 NJ w ..: a column's words are expanded by one wave only, into
 // registers, straight from registers (no LDS), one 16-byte load per column
-// and 4 steps.  A tiles go from global memory straight to LDS through a ring
+// and group.  A tiles go from global memory straight to LDS through a ring
 // of 4 stages issued 3 steps ahead; 16-byte chunk c of row r is stored at
 // chunk c ^ swz(r), swz(r) = (r ^ (r >> 3)) & 7 (no bank conflicts).  Vector
 // loads complete in issue order, and each step issues the same loads on
 // every path (clamped addresses): W = a group's word loads, F = a fill,
-//   W0 F0 F1 F2 | step 0: W1 F3 | step 1: F4 | step 2: F5 | step 3: F6 | ...
-// so before step ks (q = ks % 4) F(ks) has landed once at most 2 fills, and
-// for q = 1, 2 also the next group's words, are outstanding.
-template <int MI, int NJ, typename WordsFn, typename BoundaryFn>
+//   SPLIT: W0 F0 F1 F2 | step 0: W1 F3 | step 1: F4 | step 2: F5 | step 3: F6 | ...
+//   else:  W0 F0 W1 F1 F2 | step 0: W2 F3 | step 1: F4 | step 2: W3 F5 | step 3: F6 | ...
+// so before step ks F(ks) has landed once at most 2 fills and the words
+// issued since are outstanding (SPLIT: those of steps ks % 4 = 1, 2; else of
+// every step).  With GB each F is led by a load of the 64 g values of the
+// step after it, lane k's; they go to one of two LDS buffers as bf16 when
+// that F is waited for (all of a part's g in LDS cost the 64-row tiles their
+// fourth block per CU: 816 tiles of 4096 columns 85 us, with the buffers 66).
+template <bool SPLIT, bool GB, int MI, int NJ, typename WordsFn, typename BoundaryFn>
 __device__ __forceinline__ void sg_mainloop(const uint16_t* const (&src)[MI], int n, int g0, WordsFn&& words,
                                             BoundaryFn&& boundary, const uint32_t (&kone)[NJ],
-                                            f32x16 (&acc)[MI][NJ], int tid) {
+                                            f32x16 (&acc)[MI][NJ], int tid, const float* __restrict__ gk = nullptr) {
+  static_assert(!(SPLIT && GB), "split planes carry g themselves");
   typedef __attribute__((address_space(3))) void* lds_ptr_t;
   typedef __attribute__((address_space(1))) void* glb_ptr_t;
   constexpr int TILE = 32 * MI * 64;  // elements per stage
+  constexpr int GPI = SPLIT ? 1 : 2;  // groups of words per 4 steps
   __shared__ __attribute__((aligned(16))) uint16_t st0[TILE];
   __shared__ __attribute__((aligned(16))) uint16_t st1[TILE];
   __shared__ __attribute__((aligned(16))) uint16_t st2[TILE];
   __shared__ __attribute__((aligned(16))) uint16_t st3[TILE];
+  __shared__ __attribute__((aligned(16))) uint16_t gs[2][GB ? 64 : 1];
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lr = lane & 31, lh = lane >> 5;
   uint32_t kmask = 0x80008000u;
   asm volatile("" : "+v"(kmask));
-  // element offset of 16-byte chunk c of the lane's row in subtile 0; rows 32 i
-  // + lr swizzle by swz(lr) ^ (4 i & 7), so subtile 1 reads chunk c ^ 4's place
+  // element offset of 16-byte chunk 2 c + lh of the lane's row in subtile 0; rows
+  // 32 i + lr swizzle by swz(lr) ^ (4 i & 7), so odd subtiles read chunk ^ 4's place
   const int swz = (lr ^ (lr >> 3)) & 7;
   int off[4];
 #pragma unroll
   for (int c = 0; c < 4; ++c) off[c] = lr * 64 + (((2 * c + lh) ^ swz) << 3);
-  auto fill = [&](int f, uint16_t* st) {
+  auto g_at = [&](int f) { return GB ? gk[64 * min(f, n - 1) + lane] : 0.f; };
+  // the empty asm pins the value's first use to its step (see the words below)
+  auto put_g = [&](int f, float v) {
+    if constexpr (GB) {
+      asm volatile("" : "+v"(v));
+      if (wave == 0) gs[f & 1][lane] = f32_to_bf16(v);
+    }
+  };
+  float gr[4];  // g of step f + 1, loaded with fill(f), at f % 4
+  auto fill = [&](int f, uint16_t* st, float& gn) {
+    gn = g_at(f + 1);
     const int64_t at = int64_t(min(f, n - 1)) * 64;
 #pragma unroll
     for (int j = 0; j < MI; ++j)
       __builtin_amdgcn_global_load_lds((glb_ptr_t)(src[j] + at), (lds_ptr_t)(st + (wave * MI + j) * 512), 16, 0, 0);
   };
-  u32x4 wc[NJ], wn[NJ];
-  auto compute = [&](const uint16_t* a, int q) {
-    uint32_t w[NJ];
+  u32x4 wc[GPI][NJ], wn[GPI][NJ];
+  auto compute = [&](const uint16_t* a, int ks, int q) {
+    if constexpr (SPLIT) {
+      uint32_t w[NJ];
 #pragma unroll
-    for (int j = 0; j < NJ; ++j) w[j] = wc[j][q] >> (8 * lh);
+      for (int j = 0; j < NJ; ++j) w[j] = wc[0][j][q] >> (8 * lh);
 #pragma unroll
-    for (int s = 0; s < 2; ++s) {
-      bf16x8 b[NJ];
+      for (int s = 0; s < 2; ++s) {
+        bf16x8 b[NJ];
 #pragma unroll
-      for (int j = 0; j < NJ; ++j) b[j] = signs_to_bf16x8(w[j], 2 * s, kmask, kone[j]);
+        for (int j = 0; j < NJ; ++j) b[j] = signs_to_bf16x8(w[j], 2 * s, kmask, kone[j]);
 #pragma unroll
-      for (int pl = 0; pl < 2; ++pl)
+        for (int pl = 0; pl < 2; ++pl)
+#pragma unroll
+          for (int i = 0; i < MI; ++i) {
+            const bf16x8 f = *reinterpret_cast<const bf16x8*>(a + 2048 * i + off[(2 * pl + s) ^ (2 * (i & 1))]);
+#pragma unroll
+            for (int j = 0; j < NJ; ++j)
+              acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f, b[j], acc[i][j], 0, 0, 0);
+          }
+      }
+    } else {
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        u32x4 gv = {};
+        if constexpr (GB) gv = *reinterpret_cast<const u32x4*>(&gs[ks & 1][16 * s + 8 * lh]);
+        bf16x8 b[NJ];
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) {
+          const uint32_t w = wc[q >> 1][j][2 * (q & 1) + (s >> 1)] >> (8 * lh);
+          b[j] = GB ? signs_times_bf16x8(w, 2 * (s & 1), kmask, gv) : signs_to_bf16x8(w, 2 * (s & 1), kmask, kone[j]);
+        }
 #pragma unroll
         for (int i = 0; i < MI; ++i) {
-          // chunk 2 s + lh of plane pl: off[2 pl + s], planes swapped in odd subtiles
-          const bf16x8 f = *reinterpret_cast<const bf16x8*>(a + 2048 * i + off[2 * (pl ^ (i & 1)) + s]);
+          const bf16x8 f = *reinterpret_cast<const bf16x8*>(a + 2048 * i + off[s ^ (2 * (i & 1))]);
 #pragma unroll
-          for (int j = 0; j < NJ; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f, b[j], acc[i][j], 0, 0, 0);
+          for (int j = 0; j < NJ; ++j)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f, b[j], acc[i][j], 0, 0, 0);
         }
+      }
     }
   };
-  auto arrive = [&](auto newer) {
-    __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(decltype(newer)::value));
+  auto load_words = [&](int g, u32x4 (&w)[NJ]) {
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) w[j] = words(g0 + g, j);
+  };
+  // step ks = 4 it + q on stage `cur`, refilling `nxt` (the stage of step ks - 1)
+  auto step = [&](auto qc, int ks, const uint16_t* cur, uint16_t* nxt) {
+    constexpr int q = decltype(qc)::value;
+    constexpr int newer = 2 * (MI + (GB ? 1 : 0)) + (SPLIT ? (q == 1 || q == 2 ? NJ : 0) : NJ);
+    __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(newer));
     asm volatile("" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
+    constexpr bool first = SPLIT ? q == 0 : (q & 1) == 0;  // the first step of a group
+    constexpr int h = SPLIT ? 0 : q >> 1;
+    const int g = (ks >> 2) * GPI + h;
+    if constexpr (first) load_words(g + GPI, wn[h]);
+    put_g(ks + 1, gr[q]);
+    fill(ks + 3, nxt, gr[(q + 3) & 3]);
+    if constexpr (first) {
+      // pins the words' first use to their group: hoisted past a barrier it
+      // would wait for every load in flight
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) asm volatile("" : "+v"(wc[h][j]));
+      boundary(g0 + g, wc[h]);
+    }
+    compute(cur, ks, q);
   };
-  typedef std::integral_constant<int, 2 * MI> Fills;
-  typedef std::integral_constant<int, 2 * MI + NJ> FillsWords;
-  // pins the words' first use to their group: hoisted past a barrier it
-  // would wait for every load in flight
-  auto group = [&](int ks, const uint16_t* cur, uint16_t* nxt) {
-    arrive(Fills{});
-#pragma unroll
-    for (int j = 0; j < NJ; ++j) wn[j] = words(g0 + (ks >> 2) + 1, j);
-    fill(ks + 3, nxt);
-#pragma unroll
-    for (int j = 0; j < NJ; ++j) asm volatile("" : "+v"(wc[j]));
-    boundary(g0 + (ks >> 2), wc);
-    compute(cur, 0);
-  };
-#pragma unroll
-  for (int j = 0; j < NJ; ++j) wc[j] = words(g0, j);
+  constexpr std::integral_constant<int, 0> q0{};
+  constexpr std::integral_constant<int, 1> q1{};
+  constexpr std::integral_constant<int, 2> q2{};
+  constexpr std::integral_constant<int, 3> q3{};
+  put_g(0, g_at(0));
+  load_words(0, wc[0]);
   __builtin_amdgcn_sched_barrier(0);
-  fill(0, st0);
+  fill(0, st0, gr[0]);
   __builtin_amdgcn_sched_barrier(0);
-  fill(1, st1);
+  if constexpr (!SPLIT) {
+    load_words(1, wc[1]);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  fill(1, st1, gr[1]);
   __builtin_amdgcn_sched_barrier(0);
-  fill(2, st2);
+  fill(2, st2, gr[2]);
   __builtin_amdgcn_sched_barrier(0);
   int ks = 0;
   for (; ks + 4 <= n; ks += 4) {
-    group(ks, st0, st3);
-    arrive(FillsWords{});
-    fill(ks + 4, st0);
-    compute(st1, 1);
-    arrive(FillsWords{});
-    fill(ks + 5, st1);
-    compute(st2, 2);
-    arrive(Fills{});
-    fill(ks + 6, st2);
-    compute(st3, 3);
+    step(q0, ks, st0, st3);
+    step(q1, ks + 1, st1, st0);
+    step(q2, ks + 2, st2, st1);
+    step(q3, ks + 3, st3, st2);
 #pragma unroll
-    for (int j = 0; j < NJ; ++j) wc[j] = wn[j];
+    for (int h = 0; h < GPI; ++h)
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) wc[h][j] = wn[h][j];
   }
-  if (ks < n) group(ks, st0, st3);
-  if (ks + 1 < n) {
-    arrive(FillsWords{});
-    fill(ks + 4, st0);
-    compute(st1, 1);
-  }
-  if (ks + 2 < n) {
-    arrive(FillsWords{});
-    compute(st2, 2);
-  }
+  if (ks < n) step(q0, ks, st0, st3);
+  if (ks + 1 < n) step(q1, ks + 1, st1, st0);
+  if (ks + 2 < n) step(q2, ks + 2, st2, st1);
   // no DMA may be in flight when the block's LDS is given back
   __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(0));
   asm volatile("" ::: "memory");
@@ -323,9 +375,10 @@ __device__ __forceinline__ SgTile sg_tile(const SgParams& p) {
 }
 
 // Stage 1.  grid = row tiles * parts * column tiles.
-template <int MI>
+template <bool SPLIT, bool GB, int MI>
 __global__ __launch_bounds__(kBlock, 4) void sg_latent_kernel(SgParams p) {
   constexpr int NJ = 1;
+  constexpr int WPS = SPLIT ? 1 : 2;  // sign words per step
   const int tid = int(threadIdx.x), lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lr = lane & 31, lh = lane >> 5;
@@ -338,9 +391,9 @@ __global__ __launch_bounds__(kBlock, 4) void sg_latent_kernel(SgParams p) {
   const int c0 = (tl.nt - G.nt0) * (128 * NJ) + 32 * NJ * wave;  // the wave's first latent row
   const int ngr = (p.KW + 3) >> 2;
   const int ga = tl.part * ngr / p.parts, gb = (tl.part + 1) * ngr / p.parts;
-  const int n = min(4 * gb, p.KW) - 4 * ga;
+  const int n = (min(4 * gb, p.KW) - 4 * ga + WPS - 1) / WPS;
   const uint16_t* src[MI];
-  sg_sources<MI>(src, p.a + G.abase + int64_t(ga) * 256, p.lda, p.M, m0, tid);
+  sg_sources<MI>(src, p.a + G.abase + int64_t(ga) * (256 / WPS), p.lda, p.M, m0, tid);
   const int64_t total = int64_t(G.R) * p.KW;
   int col[NJ];
 #pragma unroll
@@ -365,7 +418,7 @@ __global__ __launch_bounds__(kBlock, 4) void sg_latent_kernel(SgParams p) {
 #pragma unroll
     for (int i = 0; i < MI; ++i) acc[i][j] = f32x16{};
   }
-  sg_mainloop<MI, NJ>(src, n, ga, words, boundary, kone, acc, tid);
+  sg_mainloop<SPLIT, GB, MI, NJ>(src, n, ga, words, boundary, kone, acc, tid, GB ? G.g + 128 * ga : nullptr);
 #pragma unroll
   for (int j = 0; j < NJ; ++j) {
     const int r = c0 + 32 * j + lr;
@@ -379,21 +432,27 @@ __global__ __launch_bounds__(kBlock, 4) void sg_latent_kernel(SgParams p) {
         const int m = m0 + 32 * i + 8 * (q >> 2) + 4 * lh + (q & 3);
         if (m >= p.M) continue;
         if (p.parts > 1) {
-          p.part[(int64_t(tl.part) * p.M + m) * (p.ldt >> 1) + G.tcol + r] = acc[i][j][q];
-        } else {
+          p.part[(int64_t(tl.part) * p.M + m) * p.tcols + G.tcol + r] = acc[i][j][q];
+          continue;
+        }
+        const float v = live ? lv * acc[i][j][q] : 0.f;
+        if constexpr (SPLIT) {
           uint16_t h, l;
-          split1(live ? lv * acc[i][j][q] : 0.f, h, l);
+          split1(v, h, l);
           uint16_t* o = p.t + int64_t(m) * p.ldt + 2 * G.tcol + (r >> 5) * 64 + (r & 31);
           o[0] = h;
           o[32] = l;
+        } else {
+          p.t[int64_t(m) * p.ldt + G.tcol + r] = f32_to_bf16(v);
         }
       }
   }
 }
 
 // T from stage 1's parts, summed in part order.  One thread per 4 columns.
+template <bool SPLIT>
 __global__ __launch_bounds__(kBlock) void sg_reduce_t_kernel(SgParams p) {
-  const int cols = p.ldt >> 1;
+  const int cols = p.tcols;
   const int64_t i = (int64_t(blockIdx.x) * kBlock + threadIdx.x) * 4;
   if (i >= int64_t(p.M) * cols) return;
   const int m = int(i / cols), c = int(i - int64_t(m) * cols);
@@ -410,9 +469,13 @@ __global__ __launch_bounds__(kBlock) void sg_reduce_t_kernel(SgParams p) {
 #pragma unroll
   for (int e = 0; e < 4; ++e) v[e] = r + e < G.R ? s[e] * G.l[r + e] : 0.f;
   split_pairs<4>(v, hi, lo);
-  uint16_t* o = p.t + int64_t(m) * p.ldt + 2 * G.tcol + (r >> 5) * 64 + (r & 31);
-  *reinterpret_cast<u32x2*>(o) = u32x2{hi[0], hi[1]};
-  *reinterpret_cast<u32x2*>(o + 32) = u32x2{lo[0], lo[1]};
+  if constexpr (SPLIT) {
+    uint16_t* o = p.t + int64_t(m) * p.ldt + 2 * G.tcol + (r >> 5) * 64 + (r & 31);
+    *reinterpret_cast<u32x2*>(o) = u32x2{hi[0], hi[1]};
+    *reinterpret_cast<u32x2*>(o + 32) = u32x2{lo[0], lo[1]};
+  } else {
+    *reinterpret_cast<u32x2*>(p.t + int64_t(m) * p.ldt + c) = u32x2{hi[0], hi[1]};
+  }
 }
 
 // Stage 2.  grid = row tiles * column tiles (p.parts 1).  A projection's
@@ -423,7 +486,7 @@ __global__ __launch_bounds__(kBlock) void sg_reduce_t_kernel(SgParams p) {
 // operand +-2^-e (exact in bf16), e = max(0, exponent of h0 / h1): acc = 2^-e
 // (h0 S0 + h1 S1) / h1 stays within a factor 2 of the larger term, and y = (h1
 // 2^e) acc.  Where h1 is zero, or h0 / h1 past 2^126, branch 1 adds nothing.
-template <typename YT, int MI, int NJ>
+template <typename YT, bool SPLIT, int MI, int NJ>
 __global__ __launch_bounds__(kBlock, 4) void sg_expand_kernel(SgParams p) {
   const int tid = int(threadIdx.x), lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -437,9 +500,10 @@ __global__ __launch_bounds__(kBlock, 4) void sg_expand_kernel(SgParams p) {
   const int c0 = (tl.nt - P.nt0) * (128 * NJ) + 32 * NJ * wave;
   const int ng0 = P.ng[0];
   const int ngr = P.nb > 1 ? ng0 + P.ng[1] : ng0;
-  const int steps = P.nb > 1 ? 4 * ng0 + P.RW[1] : P.RW[0];
+  const int nw = P.nb > 1 ? 4 * ng0 + P.RW[1] : P.RW[0];
+  const int steps = SPLIT ? nw : (nw + 1) / 2;
   const uint16_t* src[MI];
-  sg_sources<MI>(src, p.t + 2 * P.tcol, p.ldt, p.M, m0, tid);
+  sg_sources<MI>(src, p.t + (SPLIT ? 2 : 1) * P.tcol, p.ldt, p.M, m0, tid);
   int col[NJ];
 #pragma unroll
   for (int j = 0; j < NJ; ++j) col[j] = min(c0 + 32 * j + lr, P.N - 1);
@@ -486,7 +550,7 @@ __global__ __launch_bounds__(kBlock, 4) void sg_expand_kernel(SgParams p) {
       }
     }
   };
-  sg_mainloop<MI, NJ>(src, steps, 0, words, boundary, kone, acc, tid);
+  sg_mainloop<SPLIT, false, MI, NJ>(src, steps, 0, words, boundary, kone, acc, tid);
   YT* __restrict__ y = static_cast<YT*>(P.y);
 #pragma unroll
   for (int j = 0; j < NJ; ++j) {
