@@ -2479,7 +2479,7 @@ __global__ __launch_bounds__(HD) void attn_batch_combine_kernel(AttnBatchParams 
   p.out[(size_t(qi) * p.heads + h) * HD + d] = merge_partials(pp, cstride, p.chunks, HD, d);
 }
 
-#include "attn_prefill.h"
+#include "attn_rows.h"
 
 // ---------------------------------------------------------------------------
 // Q4_0 lm_head and argmax: the tail of the reference's generate_token
@@ -4332,6 +4332,36 @@ static int attn_batch_ch(int heads, int n, int64_t start) {
   return ch;
 }
 
+// Chunks of a batched attention that attn_rows_kernel takes, 0 for
+// attn_batch_kernel.  A block of the former covers 32 (token, head) rows of a
+// kv head, so the heads of a group share its keys and values, and there are
+// chunks for about a block per CU (512 blocks: 8 to 23 % slower at 1,000
+// positions); one of the latter covers one head and up to 16 tokens per wave.
+// us with 32 heads x 128, new against old:
+//   33 tokens  at 0: 14.4 / 17.4, 300: 15.7 / 23.2, 1000: 25.6 / 27.0, 2000: 37.3 / 45.0
+//   64 tokens  at 0: 15.7 / 25.2, 1000: 27.7 / 38.1, 2000: 40.2 / 57.9
+//   24 tokens  at 0: 13.5 / 13.3, 1000: 20.2 / 19.3, 1500: 22.1 / 30.3
+//   16 tokens  at 300: 14.5 / 13.5, 1000: 20.2 / 16.0, 1500: 22.0 / 23.4, 3000: 30.5 / 34.6
+//    8 tokens  at 0: 12.6 / 8.8, 1000: 19.2 / 15.1, 1500: 21.3 / 20.0, 2000: 23.3 / 21.4
+//    2 tokens, 8 kv heads  at 40: 12.8 / 9.7, 1000: 13.9 / 13.4, 1300: 14.6 / 19.2, 3500: 18.2 / 32.4
+// so: more than 32 tokens, or many positions (times heads: what the old form's
+// blocks grow with) for groups or more than 16 tokens.  With a device start
+// the old form's grid and partials are those of the cache's end, and this one
+// divides the positions there are (25 tokens at 100 of 2,100: 15.1 / 23.0; 8
+// tokens, 8 kv heads: 17.3 / 13.5, of 8,000: 18.5 / 19.5), so the lines are others.
+static int attn_rows_chunks(int heads, int kv_heads, int n, int head_dim, int64_t start, bool device_start) {
+  const bool many =
+      int64_t(heads) * (start + n) > (device_start ? 163840 : 40960) && (heads > kv_heads || n > 16);
+  const int64_t tiles = ceil_div(int64_t(n) * (heads / kv_heads), 32) * kv_heads;
+  // (the kernel's in-tile byte offsets are 32-bit)
+  if (!(n > (device_start ? 24 : 32) || many) || tiles > (1 << 20) || int64_t(kv_heads) * head_dim > (1 << 22)) return 0;
+  const int64_t groups = ceil_div(ceil_div(start, 32) + ceil_div(n, 32), 4);  // tiles of 32, one per wave
+  // (no more than the old form's chunks: the partial buffer is sized by those)
+  const int64_t most = std::min<int64_t>(std::max<int64_t>(1, 256 / tiles),
+                                         ceil_div(start + n, attn_batch_ch(heads, n, start)));
+  return int(ceil_div(groups, ceil_div(groups, most)));
+}
+
 size_t lbk_attention_batch_partial_bytes(int heads, int n, int64_t start, int head_dim) {
   if (heads < 1 || n < 1 || start < 0 || head_dim < 1) return 0;
   // (with a device start, pass max_seq - n: the grid then covers every start)
@@ -4384,10 +4414,37 @@ int lbk_attention_batch(const float* q, const float* k, const float* v, float* k
   p.ps = 4 / p.qt;
   p.scale = scale;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const dim3 grid{unsigned(heads), unsigned(p.chunks), 1u};
-  if (head_dim == 128) hipLaunchKernelGGL(attn_batch_kernel<128>, grid, dim3(kAttnThreads), 0, s, p);
-  else hipLaunchKernelGGL(attn_batch_kernel<64>, grid, dim3(kAttnThreads), 0, s, p);
-  int rc = check_launch("attn_batch_kernel");
+  if (const int chunks = attn_rows_chunks(heads, kv_heads, n, head_dim, sgrid, start_device != nullptr)) {
+    AttnRowsParams r;
+    r.q = q;
+    r.k = k;
+    r.v = v;
+    r.kc = k_cache;
+    r.vc = v_cache;
+    r.tree = tree_mask;
+    r.part = partial;
+    r.out = out;
+    r.start_ptr = start_device;
+    r.start = start;
+    r.N = n;
+    r.heads = heads;
+    r.kvh = kv_heads;
+    r.rep = p.rep;
+    r.max_seq = max_seq;
+    r.ntile = int(ceil_div(int64_t(n) * p.rep, 32));
+    r.chunks = p.chunks = chunks;
+    r.scale = scale;
+    const dim3 grid{unsigned(int64_t(kv_heads) * r.ntile * chunks), 1u, 1u};
+    // (up to 16 tokens the old form's sums are shorter: 8 sums keep this one's error no larger)
+    auto* kernel = head_dim == 128 ? (n > 16 ? &attn_rows_kernel<128, 4> : &attn_rows_kernel<128, 8>)
+                                   : (n > 16 ? &attn_rows_kernel<64, 4> : &attn_rows_kernel<64, 8>);
+    hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s, r);
+  } else {
+    const dim3 grid{unsigned(heads), unsigned(p.chunks), 1u};
+    if (head_dim == 128) hipLaunchKernelGGL(attn_batch_kernel<128>, grid, dim3(kAttnThreads), 0, s, p);
+    else hipLaunchKernelGGL(attn_batch_kernel<64>, grid, dim3(kAttnThreads), 0, s, p);
+  }
+  int rc = check_launch("lbk_attention_batch");
   if (rc != LBK_OK) return rc;
   const dim3 cgrid{unsigned(heads), unsigned(n), 1u};
   if (head_dim == 128) hipLaunchKernelGGL(attn_batch_combine_kernel<128>, cgrid, dim3(128), 0, s, p);
@@ -4416,26 +4473,28 @@ int lbk_attention_prefill(const float* q, const float* k, const float* v, float*
   // the kernel's row numbers and in-tile byte offsets are 32-bit
   if (rows > INT_MAX - 64 || tiles * kv_heads > INT_MAX || int64_t(kv_heads) * head_dim > (1 << 22))
     return set_error(LBK_ERR_ARG, "%d tokens of %d heads (%d kv heads) are too many for one call", n, heads, kv_heads);
-  AttnPrefillParams p;
+  AttnRowsParams p;
+  memset(&p, 0, sizeof(p));
   p.q = q;
   p.k = k;
   p.v = v;
   p.kc = k_cache;
   p.vc = v_cache;
   p.out = out;
-  p.start = int(start);
+  p.start = start;
   p.N = n;
   p.heads = heads;
   p.kvh = kv_heads;
   p.rep = heads / kv_heads;
   p.max_seq = max_seq;
   p.ntile = int(tiles);
+  p.chunks = 1;
   p.scale = scale;
   hipStream_t s = static_cast<hipStream_t>(stream);
   const dim3 grid{unsigned(tiles * kv_heads), 1u, 1u};
-  if (head_dim == 128) hipLaunchKernelGGL(attn_prefill_kernel<128>, grid, dim3(256), 0, s, p);
-  else hipLaunchKernelGGL(attn_prefill_kernel<64>, grid, dim3(256), 0, s, p);
-  return check_launch("attn_prefill_kernel");
+  if (head_dim == 128) hipLaunchKernelGGL((attn_rows_kernel<128, 1>), grid, dim3(256), 0, s, p);
+  else hipLaunchKernelGGL((attn_rows_kernel<64, 1>), grid, dim3(256), 0, s, p);
+  return check_launch("attn_rows_kernel");
 }
 
 int lbk_q4_0_quantize(const float* w, int64_t rows, int64_t cols, uint8_t* qs, uint16_t* d, void* stream) {
