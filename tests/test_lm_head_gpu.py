@@ -77,6 +77,25 @@ def test_q4_first_maximum_wins(gpu):
     assert int(head.argmax(torch.from_numpy(x).to(gpu)).item()) == 40
 
 
+@pytest.mark.parametrize("hidden", [32, 2048, 4096, 8192, 16384])
+@pytest.mark.parametrize("vocab", [1, 3, 15, 16, 17, 63, 65, 130])
+def test_q4_row_groups(gpu, vocab, hidden):
+    """A wave sums 4 to 16 rows together: vocabularies that end inside, at and
+    past a wave's rows and a block's; the largest logit twice, in neighbouring
+    rows (the first wins)."""
+    rng, w = _weights(11 * vocab + hidden, vocab, hidden)
+    x = rng.standard_normal(hidden).astype(np.float32)
+    top = max(vocab - 2, 0)
+    w[top] = w[vocab - 1] = x
+    head = _head(gpu, w)
+    logits = torch.empty(vocab, device=gpu)
+    tok = head.argmax(torch.from_numpy(x).to(gpu), logits=logits)
+    torch.cuda.synchronize()
+    ref, _ = Q.generate_token_head(x, *Q.quantize_q4_0(w))
+    assert O.rel_err(logits.cpu().numpy(), ref) <= 1e-5
+    assert int(tok.item()) == top
+
+
 def test_q4_fused_final_norm(gpu):
     from littlebit_amd.lm_head import Q4LMHead
     rng, w = _weights(9, 4000, 4096)
