@@ -163,9 +163,9 @@ int lbk_linear_forward(const lbk_branch* branches, int n_branches, int64_t M,
 
 /* Bytes of workspace lbk_group_forward uses for these shapes (0 with the
  * error set if the shapes are invalid), for any output dtype and buffers.
- * For M > 64 this includes room for the stream-K partial tiles of stage 1;
- * a smaller workspace, down to the size without them, is accepted and runs
- * stage 1 on whole tiles. */
+ * For M > 64 this includes room for the partial sums of stage 1 (its k range
+ * in parts); a smaller workspace, down to the size without them, is accepted
+ * and runs stage 1 whole. */
 size_t lbk_group_workspace_bytes(const lbk_projection* projs, int n_proj,
                                  int64_t M, int64_t K);
 
