@@ -448,7 +448,7 @@ class LittleBitProjectionGroup:
                 d.residual = None
                 continue
             if r is not o:  # an output was checked above
-                _require_cuda(r, "residual")
+                _require_cuda(r, f"residuals[{i}]")
             if r.dtype != torch.float32 or r.numel() != o.numel():
                 raise RuntimeError("a residual must be float32 like its output")
             d.residual = r.data_ptr()
@@ -503,7 +503,7 @@ class ChainLink:
         _check(len(self.residuals) == len(self.projections), "one residual (or None) per projection")
         for r, p in zip(self.residuals, self.projections):
             if r is not None:
-                _require_cuda(r, "residual")
+                _require_cuda(r, f"residuals[{i}]")
                 _check(r.dtype == torch.float32 and r.numel() == p.out_features,
                        "a residual must be float32 with out_features elements")
         if rms_weight is not None:
