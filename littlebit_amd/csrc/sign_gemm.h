@@ -269,10 +269,16 @@ __device__ __forceinline__ void sg_mainloop(const uint16_t* const (&src)[MI], in
 #pragma unroll
     for (int j = 0; j < NJ; ++j) w[j] = words(g0 + g, j);
   };
-  // step ks = 4 it + q on stage `cur`, refilling `nxt` (the stage of step ks - 1)
-  auto step = [&](auto qc, int ks, const uint16_t* cur, uint16_t* nxt) {
+  // step ks = 4 it + q on stage `cur`, refilling `nxt` (the stage of step ks - 1).
+  // TAIL: one of the last n % 4 steps, which loads nothing (no step is left to
+  // read it, and the compiler drops a load that nobody reads, so it could not be
+  // counted on): F(ks) has landed once at most the fills of the 2 - q later
+  // steps are outstanding.
+  auto step = [&](auto qc, auto tailc, int ks, const uint16_t* cur, uint16_t* nxt) {
     constexpr int q = decltype(qc)::value;
-    constexpr int newer = 2 * (MI + (GB ? 1 : 0)) + (SPLIT ? (q == 1 || q == 2 ? NJ : 0) : NJ);
+    constexpr bool TAIL = decltype(tailc)::value;
+    constexpr int newer =
+        TAIL ? (2 - q) * MI : 2 * (MI + (GB ? 1 : 0)) + (SPLIT ? (q == 1 || q == 2 ? NJ : 0) : NJ);
     __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(newer));
     asm volatile("" ::: "memory");
     __builtin_amdgcn_s_barrier();
@@ -280,9 +286,9 @@ __device__ __forceinline__ void sg_mainloop(const uint16_t* const (&src)[MI], in
     constexpr bool first = SPLIT ? q == 0 : (q & 1) == 0;  // the first step of a group
     constexpr int h = SPLIT ? 0 : q >> 1;
     const int g = (ks >> 2) * GPI + h;
-    if constexpr (first) load_words(g + GPI, wn[h]);
-    put_g(ks + 1, gr[q]);
-    fill(ks + 3, nxt, gr[(q + 3) & 3]);
+    if constexpr (first && !TAIL) load_words(g + GPI, wn[h]);
+    if constexpr (!TAIL || q < 2) put_g(ks + 1, gr[q]);
+    if constexpr (!TAIL) fill(ks + 3, nxt, gr[(q + 3) & 3]);
     if constexpr (first) {
       // pins the words' first use to their group: hoisted past a barrier it
       // would wait for every load in flight
@@ -311,18 +317,18 @@ __device__ __forceinline__ void sg_mainloop(const uint16_t* const (&src)[MI], in
   __builtin_amdgcn_sched_barrier(0);
   int ks = 0;
   for (; ks + 4 <= n; ks += 4) {
-    step(q0, ks, st0, st3);
-    step(q1, ks + 1, st1, st0);
-    step(q2, ks + 2, st2, st1);
-    step(q3, ks + 3, st3, st2);
+    step(q0, std::false_type{}, ks, st0, st3);
+    step(q1, std::false_type{}, ks + 1, st1, st0);
+    step(q2, std::false_type{}, ks + 2, st2, st1);
+    step(q3, std::false_type{}, ks + 3, st3, st2);
 #pragma unroll
     for (int h = 0; h < GPI; ++h)
 #pragma unroll
       for (int j = 0; j < NJ; ++j) wc[h][j] = wn[h][j];
   }
-  if (ks < n) step(q0, ks, st0, st3);
-  if (ks + 1 < n) step(q1, ks + 1, st1, st0);
-  if (ks + 2 < n) step(q2, ks + 2, st2, st1);
+  if (ks < n) step(q0, std::true_type{}, ks, st0, st3);
+  if (ks + 1 < n) step(q1, std::true_type{}, ks + 1, st1, st0);
+  if (ks + 2 < n) step(q2, std::true_type{}, ks + 2, st2, st1);
   // no DMA may be in flight when the block's LDS is given back
   __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(0));
   asm volatile("" ::: "memory");
