@@ -110,9 +110,14 @@ def deterministic(on: bool = True):
         set_deterministic(prev)
 
 
+def _stream_handle(index: int) -> int:
+    return torch.cuda.current_stream(index).cuda_stream
+
+
 # The handle of a device's current stream without the Stream object around it
-# (2 us a call, of the 8 that a one-row call spends in Python).
-_raw_stream = torch._C._cuda_getCurrentRawStream
+# (2 us a call, of the 8 that a one-row call spends in Python).  torch builds
+# without GPU support have no such function (packers and converters run there).
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", _stream_handle)
 
 
 def _ws_key(device: torch.device, stream: int) -> Tuple[int, int]:
