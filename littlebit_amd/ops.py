@@ -506,7 +506,7 @@ class ChainLink:
         self.outs = list(outs)
         self.residuals = list(residuals) if residuals is not None else [None] * len(self.projections)
         _check(len(self.residuals) == len(self.projections), "one residual (or None) per projection")
-        for r, p in zip(self.residuals, self.projections):
+        for i, (r, p) in enumerate(zip(self.residuals, self.projections)):
             if r is not None:
                 _require_cuda(r, f"residuals[{i}]")
                 _check(r.dtype == torch.float32 and r.numel() == p.out_features,
