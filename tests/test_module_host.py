@@ -2,6 +2,8 @@
 bookkeeping of quantization/modules/littlebit.py:50-93, packed state-dict
 format (:307-345), both checkpoint layouts, and the conversion invariants the
 reference test pins (test_cpu_draft.py:75-97)."""
+from types import SimpleNamespace
+
 import numpy as np
 import pytest
 import torch
@@ -158,6 +160,16 @@ def test_forward_refuses_cpu_and_unbinarised():
     m.load_state_dict(_hf_packed_state("", rng, 32, 16, [8]), strict=False)
     with pytest.raises(RuntimeError, match="GPU"):
         m(torch.zeros(1, 32))
+
+
+def test_projection_is_kept_where_the_words_are_a_parameter():
+    """A module whose U_packed a program made a parameter (nn.Module then drops the buffer) still runs."""
+    m = _convert(64, 32, split_dim=8)
+    m.set_packed_branch("main", torch.zeros(32, 1, dtype=torch.int32), torch.zeros(8, 2, dtype=torch.int32),
+                        torch.ones(1, 32), torch.ones(1, 64), mid=torch.ones(1, 8))
+    m.U_packed = nn.Parameter(m.U_packed, requires_grad=False)
+    m._proj = kept = SimpleNamespace(device=m.U_packed.device)
+    assert m._projection() is kept
 
 
 def test_from_packed_runtime_branches_has_no_meta_tensors():
