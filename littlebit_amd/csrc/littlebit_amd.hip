@@ -3740,7 +3740,9 @@ int run_group(const ProjDesc* pd, int np, int64_t M, int64_t K, const void* x, i
               int y_dtype, const Plan& pl, void* workspace, size_t workspace_bytes, void* stream) {
   if (M == 0) return LBK_OK;
   int rc = LBK_OK;
-  if (!workspace || workspace_bytes < pl.ws_min)
+  // on the GEMM path a bf16 call needs one plane, not the two that a query
+  // allows for (forward_gemm checks what its call needs)
+  if (!workspace || (workspace_bytes < pl.ws_min && (pl.mfma || x_dtype == LBK_F32)))
     return set_error(LBK_ERR_WORKSPACE, "workspace of %zu bytes needed, %zu given", pl.ws_min, workspace_bytes);
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (pl.chunk > 0 && !pl.seq) {

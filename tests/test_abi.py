@@ -199,21 +199,6 @@ def test_group_workspace_query():
     assert lib.lbk_linear_workspace_bytes(br, 2, 0, 4096, 4096) > 0
 
 
-def test_gemm_path_minimum_workspace_is_the_same_for_both_dtypes():
-    """A query covers any dtype, so the smallest accepted workspace (the size
-    without stage 1's parts) does too; a smaller one is refused before a launch."""
-    import littlebit_amd._lib as L
-    lib = L.load()
-    arr, keep = _group(2, rank=205, N=4096)
-    call = lambda dtype, n: lib.lbk_group_forward_ex(arr, 2, 100, 4096, 0x1000, dtype, None, L.LBK_F32, 0x1000, n, None)  # noqa: E731
-    assert call(L.LBK_F32, 1 << 16) == L.LBK_ERR_WORKSPACE
-    need = int(re.search(r"of (\d+) bytes needed", L.last_error()).group(1))
-    assert need <= lib.lbk_group_workspace_bytes(arr, 2, 100, 4096)
-    for dtype in (L.LBK_F32, L.LBK_BF16):
-        assert call(dtype, need - 1) == L.LBK_ERR_WORKSPACE
-        assert f"of {need} bytes needed" in L.last_error()
-
-
 def test_deterministic_mode_switch_and_workspace():
     import littlebit_amd._lib as L
     lib = L.load()
