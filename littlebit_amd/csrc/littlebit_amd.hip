@@ -3527,8 +3527,9 @@ int forward_gemm(const ProjDesc* pd, int np, int64_t M, int64_t K, const void* x
     P.tcol = tcol;
     P.nt0 = int(nt2);
     nt2 += ceil_div(pd[q].N, 128 * sp.nj2);
+    const int first = pd[q].nb > 1 && pd[q].br[1].rank > pd[q].br[0].rank ? 1 : 0;  // (see sg_expand_kernel)
     for (int b = 0; b < pd[q].nb; ++b, ++si) {
-      const lbk_branch& B = pd[q].br[b];
+      const lbk_branch& B = pd[q].br[b ^ first];
       SgSeg& S = p.seg[si];
       S.V = reinterpret_cast<const uint32_t*>(B.v_sign);
       S.Vt = reinterpret_cast<const uint32_t*>(B.v_sign_tiled);

@@ -160,7 +160,8 @@ __global__ __launch_bounds__(kBlock) void sg_scale_kernel(SgParams p) {
   }
 }
 
-// acc[i][j] += A[m0 + 32 i + .., steps 0 .. n) . S[.., c + 32 j + ..]
+// acc[.][i][j] += A[m0 + 32 i + .., steps 0 .. n) . S[.., c + 32 j + ..], the
+// lo plane's products into acc[NP - 1] (NP 2: a set of sums for each plane)
 // A: rows of 128-byte steps, `src` the lane's DMA sources of step 0; words(g)
 // loads the lane's columns' sign words of group g0 + g (4 words: 4 steps of
 // one word with SPLIT, 2 steps of two without); boundary(g) runs before group
@@ -182,10 +183,10 @@ __global__ __launch_bounds__(kBlock) void sg_scale_kernel(SgParams p) {
 // step after it, lane k's; they go to one of two LDS buffers as bf16 when
 // that F is waited for (all of a part's g in LDS cost the 64-row tiles their
 // fourth block per CU: 816 tiles of 4096 columns 85 us, with the buffers 66).
-template <bool SPLIT, bool GB, int MI, int NJ, typename WordsFn, typename BoundaryFn>
+template <bool SPLIT, bool GB, int MI, int NJ, int NP, typename WordsFn, typename BoundaryFn>
 __device__ __forceinline__ void sg_mainloop(const uint16_t* const (&src)[MI], int n, int g0, WordsFn&& words,
                                             BoundaryFn&& boundary, const uint32_t (&kone)[NJ],
-                                            f32x16 (&acc)[MI][NJ], int tid, const float* __restrict__ gk = nullptr) {
+                                            f32x16 (&acc)[NP][MI][NJ], int tid, const float* __restrict__ gk = nullptr) {
   static_assert(!(SPLIT && GB), "split planes carry g themselves");
   typedef __attribute__((address_space(3))) void* lds_ptr_t;
   typedef __attribute__((address_space(1))) void* glb_ptr_t;
@@ -241,7 +242,7 @@ __device__ __forceinline__ void sg_mainloop(const uint16_t* const (&src)[MI], in
             const bf16x8 f = *reinterpret_cast<const bf16x8*>(a + 2048 * i + off[(2 * pl + s) ^ (2 * (i & 1))]);
 #pragma unroll
             for (int j = 0; j < NJ; ++j)
-              acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f, b[j], acc[i][j], 0, 0, 0);
+              acc[pl % NP][i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f, b[j], acc[pl % NP][i][j], 0, 0, 0);
           }
       }
     } else {
@@ -260,7 +261,7 @@ __device__ __forceinline__ void sg_mainloop(const uint16_t* const (&src)[MI], in
           const bf16x8 f = *reinterpret_cast<const bf16x8*>(a + 2048 * i + off[s ^ (2 * (i & 1))]);
 #pragma unroll
           for (int j = 0; j < NJ; ++j)
-            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f, b[j], acc[i][j], 0, 0, 0);
+            acc[0][i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f, b[j], acc[0][i][j], 0, 0, 0);
         }
       }
     }
@@ -380,7 +381,11 @@ __device__ __forceinline__ SgTile sg_tile(const SgParams& p) {
   return t;
 }
 
-// Stage 1.  grid = row tiles * parts * column tiles.
+// Stage 1.  grid = row tiles * parts * column tiles.  SPLIT sums the planes
+// apart and adds the two sums at the end: half the roundings at the sums' full
+// size (4096 -> 4096, ranks 205 + 1843, M = 300: error against 64 bits 3.490e-6
+// -> 3.482e-6 of the result's norm; 1,024 rows 3.502e-6 -> 3.477e-6), no slower
+// (layer of 700 rows 818 -> 810 us).
 template <bool SPLIT, bool GB, int MI>
 __global__ __launch_bounds__(kBlock, 4) void sg_latent_kernel(SgParams p) {
   constexpr int NJ = 1;
@@ -415,16 +420,25 @@ __global__ __launch_bounds__(kBlock, 4) void sg_latent_kernel(SgParams p) {
       for (int j = 0; j < NJ; ++j) w[j] = sg_shift_words(w[j], int64_t(col[j]) * p.KW + 4 * g, total);
     }
   };
-  f32x16 acc[MI][NJ];
+  constexpr int NP = SPLIT ? 2 : 1;
+  f32x16 acc[NP][MI][NJ];
   uint32_t kone[NJ];
 #pragma unroll
   for (int j = 0; j < NJ; ++j) {
     kone[j] = 0x3F803F80u;
     asm volatile("" : "+v"(kone[j]));
 #pragma unroll
-    for (int i = 0; i < MI; ++i) acc[i][j] = f32x16{};
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+      for (int u = 0; u < NP; ++u) acc[u][i][j] = f32x16{};
   }
-  sg_mainloop<SPLIT, GB, MI, NJ>(src, n, ga, words, boundary, kone, acc, tid, GB ? G.g + 128 * ga : nullptr);
+  sg_mainloop<SPLIT, GB, MI, NJ, NP>(src, n, ga, words, boundary, kone, acc, tid, GB ? G.g + 128 * ga : nullptr);
+  if constexpr (NP == 2) {
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) acc[0][i][j] += acc[1][i][j];
+  }
 #pragma unroll
   for (int j = 0; j < NJ; ++j) {
     const int r = c0 + 32 * j + lr;
@@ -438,10 +452,10 @@ __global__ __launch_bounds__(kBlock, 4) void sg_latent_kernel(SgParams p) {
         const int m = m0 + 32 * i + 8 * (q >> 2) + 4 * lh + (q & 3);
         if (m >= p.M) continue;
         if (p.parts > 1) {
-          p.part[(int64_t(tl.part) * p.M + m) * p.tcols + G.tcol + r] = acc[i][j][q];
+          p.part[(int64_t(tl.part) * p.M + m) * p.tcols + G.tcol + r] = acc[0][i][j][q];
           continue;
         }
-        const float v = live ? lv * acc[i][j][q] : 0.f;
+        const float v = live ? lv * acc[0][i][j][q] : 0.f;
         if constexpr (SPLIT) {
           uint16_t h, l;
           split1(v, h, l);
@@ -487,7 +501,10 @@ __global__ __launch_bounds__(kBlock) void sg_reduce_t_kernel(SgParams p) {
 // Stage 2.  grid = row tiles * column tiles (p.parts 1).  A projection's
 // steps are branch 0's words, padded to whole groups of 4 (the T columns
 // there are zero, whatever bits the words hold), then branch 1's: one
-// pipeline through both.  One accumulator set: after branch 0 each column's
+// pipeline through both.  Branch 0 is the one of the larger rank: the other's
+// few products are the ones rounded at the size of the whole sum (error
+// against 64 bits at the shape above 3.482e-6, 3.492e-6 in the other order and
+// 3.480e-6 with a call per branch).  One accumulator set: after branch 0 each column's
 // S0 is scaled by r = (h0 / h1) 2^-e in fp32 and branch 1 is added with the
 // operand +-2^-e (exact in bf16), e = max(0, exponent of h0 / h1): acc = 2^-e
 // (h0 S0 + h1 S1) / h1 stays within a factor 2 of the larger term, and y = (h1
@@ -519,7 +536,7 @@ __global__ __launch_bounds__(kBlock, 4) void sg_expand_kernel(SgParams p) {
     const int64_t rw = b ? P.RW[1] : P.RW[0];
     return sg_load_words(b ? P.U[1] : P.U[0], int64_t(col[j]) * rw + 4 * gl, int64_t(P.N) * rw);
   };
-  f32x16 acc[MI][NJ];
+  f32x16 acc[1][MI][NJ];
   uint32_t kone[NJ];
   float f[NJ];
 #pragma unroll
@@ -528,7 +545,7 @@ __global__ __launch_bounds__(kBlock, 4) void sg_expand_kernel(SgParams p) {
     asm volatile("" : "+v"(kone[j]));
     f[j] = P.h[0][col[j]];
 #pragma unroll
-    for (int i = 0; i < MI; ++i) acc[i][j] = f32x16{};
+    for (int i = 0; i < MI; ++i) acc[0][i][j] = f32x16{};
   }
   auto boundary = [&](int g, u32x4 (&w)[NJ]) {
     const int b = g >= ng0 ? 1 : 0, gl = g - (b ? ng0 : 0);
@@ -546,7 +563,7 @@ __global__ __launch_bounds__(kBlock, 4) void sg_expand_kernel(SgParams p) {
         if (h1 != 0.f && e <= 126) {
           const float r = ldexpf(ratio, -e);
 #pragma unroll
-          for (int i = 0; i < MI; ++i) acc[i][j] *= r;
+          for (int i = 0; i < MI; ++i) acc[0][i][j] *= r;
           f[j] = ldexpf(h1, e);
           kone[j] = (0x3F80u - (uint32_t(e) << 7)) * 0x10001u;
         } else {
@@ -556,7 +573,7 @@ __global__ __launch_bounds__(kBlock, 4) void sg_expand_kernel(SgParams p) {
       }
     }
   };
-  sg_mainloop<SPLIT, false, MI, NJ>(src, steps, 0, words, boundary, kone, acc, tid);
+  sg_mainloop<SPLIT, false, MI, NJ, 1>(src, steps, 0, words, boundary, kone, acc, tid);
   YT* __restrict__ y = static_cast<YT*>(P.y);
 #pragma unroll
   for (int j = 0; j < NJ; ++j) {
@@ -571,7 +588,7 @@ __global__ __launch_bounds__(kBlock, 4) void sg_expand_kernel(SgParams p) {
         const int m = m0 + 32 * i + 8 * (q >> 2) + 4 * lh + (q & 3);
         if (m >= p.M) continue;
         const size_t o = size_t(m) * P.N + nn;
-        store_out(y, o, f[j] * acc[i][j][q] + bn + (res ? res[o] : 0.f));
+        store_out(y, o, f[j] * acc[0][i][j][q] + bn + (res ? res[o] : 0.f));
       }
   }
 }

@@ -113,3 +113,31 @@ def test_sign_gemm_scale_ratios(gpu):
         err = np.abs(y - ref).max(0) / np.abs(ref).max(0)
         print(f"[split] ratios scale={scale:g} worst column {err.max():.2e}", flush=True)
         assert np.isfinite(y).all() and err.max() <= TOL[torch.float32]
+
+
+@pytest.mark.parametrize("M", [70, 300, 1024])
+def test_two_branches_are_as_exact_as_a_call_each(gpu, M):
+    """Both branches of a call share one set of sums in stage 2.  The branch
+    of the smaller rank comes second, whatever order the caller has them in:
+    its 7 words' 28 MFMAs and the rescale round at the size of the whole sum,
+    sqrt(30) * 2**-24 / sqrt(3) = 1.9e-7 of it at most beside 3.5e-6 from the
+    planes, 0.15 % in quadrature (1,843 columns second: 0.3 to 0.6 %)."""
+    from littlebit_amd import LittleBitProjection
+    K, N, ranks = 4096, 4096, [205, 1843]
+    joined, apart = [], []
+    for seed in (9700, 9701):
+        _, grp, x = _make(gpu, seed, M, K, [(N, ranks)], torch.float32)
+        brs = grp.projections[0].branches
+        for b, r in zip(brs, ranks):
+            b.mid.div_(r ** 0.5)  # branches of equal size, as in a trained model
+        pm1 = lambda w, n: (1 - 2 * ((w.unsqueeze(-1) >> torch.arange(32, dtype=torch.int32, device=gpu)) & 1)  # noqa: E731
+                            ).reshape(w.shape[0], -1)[:, :n].double()
+        ref = sum(((x.double() * b.v2.double()) @ pm1(b.v_sign, K).t().contiguous() * b.mid.double())
+                  @ pm1(b.u_sign, b.mid.numel()).t().contiguous() * b.u1.double() for b in brs)
+        err = lambda y: float((y.double() - ref).norm() / ref.norm())  # noqa: E731
+        y = LittleBitProjection(brs).forward(x)
+        assert torch.equal(y, LittleBitProjection(brs[::-1]).forward(x)), "the caller's order changes nothing"
+        joined.append(err(y))
+        apart.append(err(sum(LittleBitProjection([b]).forward(x) for b in brs)))
+    print(f"[split] M={M} joined {joined} apart {apart}", flush=True)
+    assert sum(joined) <= 1.002 * sum(apart)
