@@ -2959,9 +2959,11 @@ size_t gemm_ws_bytes(const ProjDesc* pd, int np, int64_t M, int64_t K, int plane
 //   768 tiles of 32 rows and 100.1 us in 384 whole tiles of 64).
 //   Stage 2: 32 x 128 tiles while they are few (fp32, M = 512, 4096 columns:
 //   512 tiles 22.2 us, 64 x 128 27.1 us, 64 x 256 43.8 us) or the ranks are
-//   short (each tile then mostly stores y), 64 x 256 where those give 600
+//   short (each tile then mostly stores y; as long as a launch holds the
+//   blocks: 2**23 rows x 8192 columns are 2**24 of them), 64 x 256 where those give 600
 //   blocks (fp32, M = 1024, gate and up: 217.6 us against 227.4 us as 64 x 128
 //   and 251.5 us as 32 x 128; bf16 141.3, 146.0, 174.6 us), else 64 x 128.
+constexpr int64_t kMaxLaunchBlocks = (int64_t(1) << 32) / kBlock - 1;  // a grid's threads are counted in 32 bits
 struct SgPlan {
   int mi1, parts;  // stage 1: 32 mi1 rows x 128 columns, parts of the k range
   int mi2, nj2;    // stage 2: 32 mi2 rows x 128 nj2 columns
@@ -2998,7 +3000,8 @@ SgPlan sg_plan(const ProjDesc* pd, int np, int64_t M, int64_t K, bool split) {
   s.parts = int(std::max<int64_t>(1, std::min<int64_t>({parts, 8, ceil_div(K, 128) / 2})));
   s.part_bytes = s.parts > 1 ? size_t(s.parts) * size_t(M) * size_t(cols) * sizeof(float) : 0;
   s.mi2 = s.nj2 = 1;
-  if (ceil_div(M, 32) * c2 > (split ? 1100 : 800) && steps > 16) {
+  const int64_t tiles = ceil_div(M, 32) * c2;
+  if (tiles > (split ? 1100 : 800) && (steps > 16 || tiles > kMaxLaunchBlocks)) {
     s.mi2 = 2;
     s.nj2 = ceil_div(M, 64) * c2w >= 600 ? 2 : 1;
   }
@@ -3561,7 +3564,7 @@ int forward_gemm(const ProjDesc* pd, int np, int64_t M, int64_t K, const void* x
   const int64_t blocks1 = ceil_div(M, 32 * sp.mi1) * nt1 * sp.parts, blocks2 = ceil_div(M, 32 * sp.mi2) * nt2;
   int64_t nt128 = 0;
   for (int q = 0; q < np; ++q) nt128 += ceil_div(pd[q].N, 128);
-  if (nt1 > 65535 || nt128 > 65535 || blocks1 > INT_MAX || blocks2 > INT_MAX)
+  if (nt1 > 65535 || nt128 > 65535 || blocks1 > kMaxLaunchBlocks || blocks2 > kMaxLaunchBlocks)
     return set_error(LBK_ERR_ARG, "too many column tiles for the GEMM path");
 
   int rc;

@@ -2,15 +2,56 @@
 // AddressSanitizer and UndefinedBehaviorSanitizer on the host pass only
 // (tests/test_host_sanitizers.py).  It makes no device call: workspace
 // queries (which run the whole launch planning: path choice, row chunks,
-// expand shapes, stream-K sizing) over a grid of shapes, and every argument
-// error the entry points return before a launch.  Factor pointers are fake
-// aligned addresses that the host code never dereferences.
+// expand shapes, stage 1's parts) over a grid of shapes, every argument error
+// the entry points return before a launch, and the launches of calls on the
+// GEMM path, which this program records instead of the runtime (its own
+// hipLaunchKernel).  Factor pointers are fake aligned addresses that the host
+// code never dereferences.
+#include <hip/hip_runtime.h>
+
 #include <cstdint>
 #include <cstdio>
 #include <cstring>
+#include <map>
+#include <string>
 #include <vector>
 
 #include "littlebit_amd.h"
+
+// ---- the runtime's launch entry points, recorded
+struct Launch {
+  std::string name;  // mangled
+  dim3 grid, block;
+};
+static std::vector<Launch> launches;
+static std::map<const void*, std::string>& kernel_names() {
+  static std::map<const void*, std::string> names;  // (used by other files' static constructors)
+  return names;
+}
+extern "C" {
+void __hipRegisterFunction(void**, const void* host, char*, const char* name, unsigned, void*, void*, void*, void*,
+                           int*) {
+  kernel_names()[host] = name;
+}
+static dim3 pushed[2];  // a launch's shape goes through these two
+hipError_t __hipPushCallConfiguration(dim3 grid, dim3 block, size_t, hipStream_t) {
+  pushed[0] = grid;
+  pushed[1] = block;
+  return hipSuccess;
+}
+hipError_t __hipPopCallConfiguration(dim3* grid, dim3* block, size_t* shmem, hipStream_t* stream) {
+  *grid = pushed[0];
+  *block = pushed[1];
+  *shmem = 0;
+  *stream = nullptr;
+  return hipSuccess;
+}
+hipError_t hipLaunchKernel(const void* f, dim3 grid, dim3 block, void**, size_t, hipStream_t) {
+  launches.push_back({kernel_names()[f], grid, block});
+  return hipSuccess;
+}
+hipError_t hipGetLastError() { return hipSuccess; }
+}
 
 static int failures = 0;
 #define EXPECT(cond, ...)                         \
@@ -292,6 +333,52 @@ int main() {
     {
       lbk_chain_link bad[1] = {{&po, 0, 4096, &plain}};
       EXPECT(lbk_chain_forward(bad, 1, x0, ws, 1u << 30, nullptr) == LBK_ERR_ARG, "link without projections");
+    }
+  }
+  // ---- the GEMM path's launches: grids whose threads fit 32 bits up to the
+  // largest outputs a card holds
+  {
+    struct Case {
+      const char* test;
+      int64_t M, K;
+      int64_t spec[2][3];  // N, ranks of up to two projections
+      int x_dtype;
+      const char *latent, *expand;
+      bool parts;
+    };
+    const int F = LBK_F32, B = LBK_BF16;
+    const Case cases[] = {
+        // tall outputs of a short rank
+        {"2**23 rows", int64_t(1) << 23, 64, {{8192, 205, 0}}, B, "Lb0ELb1ELi2E", "IfLb0ELi2ELi2E", false},
+        {"2**22 rows", int64_t(1) << 22, 64, {{4096, 205, 0}}, F, "Lb1ELb0ELi2E", "IfLb1ELi1ELi1E", false},
+        {"65535 column tiles", 3000, 64, {{65535 * 128, 205, 0}}, B, "Lb0ELb1E", "IfLb0ELi1ELi1E", false},
+    };
+    for (const Case& c : cases) {
+      std::vector<lbk_branch> br;
+      for (int q = 0; q < 2 && c.spec[q][0]; ++q)
+        for (int b = 1; b < 3 && c.spec[q][b]; ++b) br.push_back(branch(c.spec[q][b], 10 * q + 5 * b));
+      std::vector<lbk_projection> pj;
+      for (int q = 0, at = 0; q < 2 && c.spec[q][0]; ++q) {
+        const int nb = c.spec[q][2] ? 2 : 1;
+        pj.push_back({br.data() + at, nb, c.spec[q][0], nullptr, const_cast<void*>(fake(90 + q)), nullptr});
+        at += nb;
+      }
+      const int np = int(pj.size());
+      launches.clear();
+      const size_t n = lbk_group_workspace_bytes(pj.data(), np, c.M, c.K);
+      const int rc = lbk_group_forward_ex(pj.data(), np, c.M, c.K, xf, c.x_dtype, nullptr, LBK_F32, ws, n, nullptr);
+      EXPECT(rc == LBK_OK, "%s: M=%lld refused", c.test, (long long)c.M);
+      bool latent = false, expand = false, parts = false;
+      for (const Launch& l : launches) {
+        std::printf("%s M=%lld: %s grid %u %u\n", c.test, (long long)c.M, l.name.c_str(), l.grid.x, l.grid.y);
+        latent = latent || l.name.find(std::string("sg_latent_kernelI") + c.latent) != std::string::npos;
+        expand = expand || l.name.find(std::string("sg_expand_kernel") + c.expand) != std::string::npos;
+        parts = parts || l.name.find("sg_reduce_t_kernel") != std::string::npos;
+        EXPECT(uint64_t(l.grid.x) * l.block.x < (uint64_t(1) << 32) && l.grid.y < 65536, "%s: %s of %u x %u blocks",
+               c.test, l.name.c_str(), l.grid.x, l.grid.y);
+      }
+      EXPECT(latent && expand && parts == c.parts, "%s: M=%lld K=%lld dtype %d runs other kernels", c.test,
+             (long long)c.M, (long long)c.K, c.x_dtype);
     }
   }
   std::printf("%s (%d failures)\n", failures ? "FAILED" : "ok", failures);
