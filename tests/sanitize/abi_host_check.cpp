@@ -233,6 +233,28 @@ int main() {
   EXPECT(lbk_attention_batch(xf, xf, xf, xf, xf, 65, 32, 8, 128, 1024, nullptr, 0, nullptr, 1.f, xf, 1 << 20, xf,
                              nullptr) == LBK_ERR_ARG,
          "batch n > 64");
+  {
+    auto prefill = [&](const float* q, float* kc, int n, int heads, int kv, int hd, int max_seq, int64_t start) {
+      return lbk_attention_prefill(q, xf, xf, kc, xf, n, heads, kv, hd, max_seq, start, 1.f, xf, nullptr);
+    };
+    const float* off = reinterpret_cast<const float*>(reinterpret_cast<uintptr_t>(xf) + 4);
+    launches.clear();
+    EXPECT(prefill(xf, xf, 0, 32, 8, 128, 1024, 0) == LBK_ERR_ARG, "prefill n 0");
+    EXPECT(prefill(xf, xf, 65, 32, 5, 128, 1024, 0) == LBK_ERR_ARG, "prefill heads not a multiple of kv_heads");
+    EXPECT(prefill(xf, xf, 65, 0, 0, 128, 1024, 0) == LBK_ERR_ARG, "prefill no heads");
+    EXPECT(prefill(xf, xf, 65, 32, 8, 96, 1024, 0) == LBK_ERR_ARG, "prefill head_dim");
+    EXPECT(prefill(xf, xf, 65, 32, 8, 128, 0, 0) == LBK_ERR_ARG, "prefill max_seq 0");
+    EXPECT(prefill(xf, xf, 65, 32, 8, 128, 1024, -1) == LBK_ERR_ARG, "prefill start < 0");
+    EXPECT(prefill(xf, xf, 65, 32, 8, 128, 1024, 960) == LBK_ERR_ARG, "prefill past the cache");
+    EXPECT(prefill(xf, xf, 65, 32, 8, 128, 1024, int64_t(1) << 62) == LBK_ERR_ARG, "prefill start huge");
+    EXPECT(prefill(nullptr, xf, 65, 32, 8, 128, 1024, 0) == LBK_ERR_ARG, "prefill NULL q");
+    EXPECT(prefill(off, xf, 65, 32, 8, 128, 1024, 0) == LBK_ERR_ARG, "prefill misaligned q");
+    EXPECT(prefill(xf, const_cast<float*>(off), 65, 32, 8, 128, 1024, 0) == LBK_ERR_ARG, "prefill misaligned cache");
+    EXPECT(prefill(xf, xf, 1 << 24, 1 << 20, 1, 64, 1 << 24, 0) == LBK_ERR_ARG, "prefill too many rows");
+    EXPECT(launches.empty(), "a refused prefill launched");
+    EXPECT(prefill(xf, xf, 65, 32, 8, 128, 1024, 959) == LBK_OK, "prefill up to the cache's end");
+    EXPECT(launches.size() == 1 && launches[0].grid.x == (65 * 4 + 31) / 32 * 8, "prefill grid");
+  }
   EXPECT(lbk_q4_0_quantize(xf, 4, 33, static_cast<uint8_t*>(ws), static_cast<uint16_t*>(ws), nullptr) == LBK_ERR_ARG,
          "q4 cols % 32");
   EXPECT(lbk_lm_head_q4_workspace_bytes(32000, 4096) > 0, "lm head workspace");
@@ -335,8 +357,8 @@ int main() {
       EXPECT(lbk_chain_forward(bad, 1, x0, ws, 1u << 30, nullptr) == LBK_ERR_ARG, "link without projections");
     }
   }
-  // ---- the GEMM path's launches: grids whose threads fit 32 bits up to the
-  // largest outputs a card holds
+  // ---- the GEMM path's launches: the forms that the GPU tests mean to reach,
+  // and grids whose threads fit 32 bits up to the largest outputs a card holds
   {
     struct Case {
       const char* test;
@@ -348,6 +370,28 @@ int main() {
     };
     const int F = LBK_F32, B = LBK_BF16;
     const Case cases[] = {
+        // tests/test_gemm_wide_gpu.py
+        {"wide scale edges", 1024, 256, {{16384, 40, 600}}, F, "Lb1ELb0E", "IfLb1ELi2ELi2E", false},
+        {"wide scale edges", 1024, 256, {{16384, 40, 600}}, B, "Lb0ELb1E", "IfLb0ELi2ELi2E", false},
+        {"wide scale edges", 1100, 256, {{5000, 40, 600}}, F, "Lb1ELb0E", "IfLb1ELi2ELi1E", false},
+        {"wide scale edges", 1100, 256, {{5000, 40, 600}}, B, "Lb0ELb1E", "IfLb0ELi2ELi1E", false},
+        {"wide group", 1100, 512, {{8192, 37, 601}, {8192, 37, 601}}, B, "Lb0ELb1E", "IfLb0ELi2ELi2E", false},
+        // tests/test_sign_gemm_gpu.py
+        {"64-row tiles in parts", 330, 8256, {{130, 205, 1843}}, F, "Lb1ELb0ELi2E", "IfLb1ELi1ELi1E", true},
+        {"64-row tiles in parts", 330, 8256, {{130, 205, 1843}}, B, "Lb0ELb1ELi2E", "IfLb0ELi1ELi1E", true},
+        {"64-row tiles, K off", 2049, 264, {{130, 205, 3000}}, F, "Lb1ELb0ELi2E", "IfLb1E", false},
+        {"64-row tiles, K off", 2049, 264, {{130, 205, 3000}}, B, "Lb0ELb0ELi2E", "IfLb0E", false},
+        {"64-row tiles, odd steps", 2049, 320, {{130, 205, 3000}}, B, "Lb0ELb1ELi2E", "IfLb0E", false},
+        {"64 x 128", 1100, 200, {{5000, 40, 600}}, F, "Lb1E", "IfLb1ELi2ELi1E", false},
+        {"64 x 256", 1100, 200, {{9000, 40, 601}}, F, "Lb1E", "IfLb1ELi2ELi2E", false},
+        {"32 x 128", 200, 260, {{4500, 40, 600}}, F, "Lb1E", "IfLb1ELi1ELi1E", false},
+        {"ratios", 72, 256, {{160, 64, 200}}, F, "Lb1E", "IfLb1ELi1ELi1E", false},
+        // tests/test_gpu_parity.py: stage 1 in parts
+        {"parts", 100, 4096, {{4096, 204, 1843}, {1024, 81, 737}}, B, "Lb0ELb1ELi1E", "IfLb0E", true},
+        {"parts", 1024, 11008, {{4096, 298, 2686}}, B, "Lb0ELb1ELi2E", "IfLb0E", true},
+        {"parts", 1024, 11008, {{4096, 298, 2686}}, F, "Lb1ELb0ELi2E", "IfLb1E", true},
+        {"parts", 300, 14336, {{4096, 318, 2867}}, B, "Lb0ELb1ELi2E", "IfLb0E", true},
+        {"parts", 129, 4096, {{1024, 130, 7}}, F, "Lb1ELb0ELi1E", "IfLb1E", true},
         // tall outputs of a short rank
         {"2**23 rows", int64_t(1) << 23, 64, {{8192, 205, 0}}, B, "Lb0ELb1ELi2E", "IfLb0ELi2ELi2E", false},
         {"2**22 rows", int64_t(1) << 22, 64, {{4096, 205, 0}}, F, "Lb1ELb0ELi2E", "IfLb1ELi1ELi1E", false},

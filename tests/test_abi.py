@@ -194,7 +194,7 @@ def test_group_workspace_query():
     assert lib.lbk_group_workspace_bytes(arr, 3, 64, 4096) == grp
     assert lib.lbk_group_workspace_bytes(arr, 3, 65, 4096) > grp  # GEMM path: per-call planes
     assert lib.lbk_group_workspace_bytes(arr, 0, 8, 4096) == 0
-    # M = 0 plans no tiles (the stream-K sizing once divided by its zero block count)
+    # M = 0 plans no tiles (a sizing rule once divided by their number)
     assert lib.lbk_group_workspace_bytes(arr, 3, 0, 4096) > 0
     assert lib.lbk_linear_workspace_bytes(br, 2, 0, 4096, 4096) > 0
 

@@ -230,22 +230,21 @@ def _min_workspace(lib, arr, n, M, K, x, x_dtype, ws, stream):
 
 
 @pytest.mark.parametrize("M,K,specs,x_dtype", [
-    (100, 4096, [(4096, [204, 1843]), (1024, [81, 737])], torch.bfloat16),  # 4 parts per tile
-    (2048, 4096, [(4096, [204, 1843])], torch.bfloat16),                    # 512 blocks, 8 XCD groups
+    (100, 4096, [(4096, [204, 1843]), (1024, [81, 737])], torch.bfloat16),  # 32-row tiles, 5 parts
+    (1024, 11008, [(4096, [298, 2686])], torch.bfloat16),                   # 64-row tiles, 2 parts
+    (1024, 11008, [(4096, [298, 2686])], torch.float32),                    # the same in hi/lo planes
     (300, 14336, [(4096, [318, 2867])], torch.bfloat16),
     (129, 4096, [(1024, [130, 7])], torch.float32),                         # hi/lo planes, scaled copy
 ])
-def test_stream_k_matches_whole_tiles(gpu, M, K, specs, x_dtype):
-    """Stage 1 of the GEMM path shares its (tile, k-step) iterations over
-    resident blocks when whole tiles would leave CUs idle (stream-K, partial
-    tiles summed by the part that completes them); given a workspace without
-    room for the partial tiles the same call runs whole tiles.  The partial
-    sums meet in another order, so the forms agree to fp32 rounding with fp32
-    activations (T kept as hi/lo bf16 planes, ~2**-17), and to 1e-3 with bf16
-    ones (T rounded to bf16: an ulp of fp32 can move a T element by 2**-8);
-    twice in a row (the tile counters are left at zero), each form bit for
-    bit the same both times (the completing part sums the parts in block
-    order); both match the oracle."""
+def test_stage1_parts_match_whole_tiles(gpu, M, K, specs, x_dtype):
+    """Stage 1 of the GEMM path cuts its k range into parts where whole tiles
+    would leave CUs idle (each part stores its fp32 sums, sg_reduce_t_kernel
+    adds them in part order); given a workspace without room for the parts the
+    same call runs whole tiles.  The partial sums meet in another order, so the
+    forms differ, and agree to fp32 rounding with fp32 activations (T kept as
+    hi/lo bf16 planes, ~2**-17), and to 1e-3 with bf16 ones (T rounded to
+    bf16: an ulp of fp32 can move a T element by 2**-8); each form is bit for
+    bit the same twice; both match the oracle."""
     import ctypes
     import littlebit_amd._lib as L
     from littlebit_amd import LittleBitProjection
@@ -260,7 +259,7 @@ def test_stream_k_matches_whole_tiles(gpu, M, K, specs, x_dtype):
     stream = torch.cuda.current_stream(gpu).cuda_stream
     dt = L.LBK_BF16 if x_dtype == torch.bfloat16 else L.LBK_F32
     results = []
-    for form in ("whole", "stream-k", "whole", "stream-k"):
+    for form in ("whole", "parts", "whole", "parts"):
         outs = [torch.full((M, N), float("nan"), device=gpu) for N, _ in specs]
         arr = (L.LbkProjection * len(projs))()
         for i, (p, o) in enumerate(zip(projs, outs)):
@@ -272,25 +271,25 @@ def test_stream_k_matches_whole_tiles(gpu, M, K, specs, x_dtype):
             arr[i].residual = None
         full = lib.lbk_group_workspace_bytes(arr, len(projs), M, K)
         ws = torch.zeros(full, dtype=torch.uint8, device=gpu)
-        n = full if form == "stream-k" else _min_workspace(lib, arr, len(projs), M, K, tx.data_ptr(), dt, ws, stream)
-        print(f"[stream-k] M={M} K={K} {form}: workspace {n} of {full}", flush=True)
+        n = full if form == "parts" else _min_workspace(lib, arr, len(projs), M, K, tx.data_ptr(), dt, ws, stream)
+        print(f"[parts] M={M} K={K} {form}: workspace {n} of {full}", flush=True)
         L.check(lib.lbk_group_forward_ex(arr, len(projs), M, K, tx.data_ptr(), dt, None, L.LBK_F32, ws.data_ptr(), n,
                                          stream), "lbk_group_forward_ex")
         torch.cuda.synchronize()
         results.append([o.cpu().numpy() for o in outs])
-    assert full > _min_workspace(lib, arr, len(projs), M, K, tx.data_ptr(), dt, ws, stream), "no stream-K form"
+    assert not all(np.array_equal(a, b) for a, b in zip(results[0], results[1])), "both ran one form"
     for a, b in zip(results[0] + results[1], results[2] + results[3]):
         assert np.array_equal(a, b), "a GEMM-path form changed between two identical calls"
     agree = 1e-3 if x_dtype == torch.bfloat16 else 1e-5
     for r in results[1:]:
         for a, b in zip(results[0], r):
             err = O.rel_err(b, a)
-            print(f"[stream-k] forms differ by {err:.2e}", flush=True)
+            print(f"[parts] forms differ by {err:.2e}", flush=True)
             assert err <= agree
     tol = TOL_BF16_PREFILL if x_dtype == torch.bfloat16 else TOL_F32
     rows = np.unique(np.r_[0:min(M, 48), max(0, M - 48):M])  # rows are independent: a sample pins the call
     for (N, _), brs, y in zip(specs, host, results[1]):
-        _check(y[rows], xu[rows], [b.as_dict() for b in brs], K, N, tol, what=f"stream-K M={M} K={K} N={N}")
+        _check(y[rows], xu[rows], [b.as_dict() for b in brs], K, N, tol, what=f"parts M={M} K={K} N={N}")
 
 
 @pytest.mark.parametrize("M,K,N,ranks", [(65, 4096, 4096, [205, 1843]), (96, 11008, 4096, [298, 2686]),

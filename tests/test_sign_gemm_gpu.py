@@ -10,9 +10,12 @@ import oracle.littlebit_oracle as O
 pytestmark = pytest.mark.gpu
 
 # hi + lo planes keep 16-17 mantissa bits of every product's activation
-# (2**-17 of its magnitude), as on the decode path; bf16 calls round x * g (or g)
-# and the latent vector to 2**-9 of their magnitudes
-TOL = {torch.float32: 1e-3, torch.bfloat16: 5e-3}
+# (2**-17 of its magnitude, in each stage), as on the decode path: the largest
+# difference over the largest result measures 3.5e-6, a few standard deviations
+# of the sums' error are 4e-5, and a branch without its lo plane shows 5.8e-4
+# (A's) or 6.8e-4 (T's).  bf16 calls round x * g (or g) and the latent vector to
+# 2**-9 of their magnitudes.
+TOL = {torch.float32: 4e-5, torch.bfloat16: 5e-3}
 
 
 def _make(gpu, seed, M, K, specs, x_dtype, tile_v=True, offset=0):
@@ -51,9 +54,10 @@ def _check(host, specs, K, x, outs, rows=None, tol=TOL[torch.float32]):
     (1100, 200, [(9000, [40, 601])]),               # stage 2 as 64 x 256 tiles, partial last tiles
     (2049, 264, [(130, [205, 3000])]),              # stage 1 as 64-row tiles
     (2049, 320, [(130, [205, 3000])]),              # the same, bf16 rows read as they are, an odd step
-    (270, 8256, [(130, [205, 1843])]),              # long rows: 64-row tiles in parts
+    (330, 8256, [(130, [205, 1843])]),              # long rows: 64-row tiles in parts
 ])
 def test_sign_gemm_edges(gpu, M, K, specs, x_dtype):
+    """(Which kernels these shapes run is checked in tests/sanitize/abi_host_check.cpp.)"""
     host, grp, x = _make(gpu, 9100 + M, M, K, specs, x_dtype)
     a = grp.forward(x, out_dtype=torch.float32)
     b = grp.forward(x, out_dtype=torch.float32)
@@ -88,13 +92,18 @@ def test_sign_gemm_inputs(gpu, M, x_dtype, offset):
     _check(host, specs, K, x, grp.forward(x, out_dtype=torch.float32))
 
 
-def test_sign_gemm_scale_ratios(gpu):
-    """Both branches share one accumulator set, rescaled by h0 / h1 between
-    them: ratios up to 2**+-60 with sums as large as their product with the
-    ratio still representable, zeros, and infinities stay where the formula
-    has them."""
-    M, K, N = 72, 256, 160
-    host, grp, x = _make(gpu, 9500, M, K, [(N, [64, 200])], torch.float32)
+@pytest.mark.parametrize("M,N,ranks", [
+    (72, 176, [64, 200]),     # stage 2 as 32 x 128 tiles
+    (1100, 5000, [40, 600]),  # 64 x 128
+    (1100, 9000, [601, 40]),  # 64 x 256
+])
+def test_sign_gemm_scale_ratios(gpu, M, N, ranks):
+    """Both branches share one accumulator set, rescaled by the ratio of
+    their row scales between them: ratios up to 2**+-60 with sums as large as
+    their product with the ratio still representable, zeros, and infinities
+    and NaN in either scale give what the formula has."""
+    K = 256
+    host, grp, x = _make(gpu, 9500, M, K, [(N, ranks)], torch.float32)
     brs = host[0]
     h0, h1 = brs[0].h, brs[1].h
     for i in range(0, 120, 2):
@@ -102,17 +111,27 @@ def test_sign_gemm_scale_ratios(gpu):
         h0[i + 1] = h1[i + 1] * np.float32(2.0 ** -(i // 2))
     h1[120:130] = 0.0
     h0[130:140] = 0.0
+    h0[160:162] = np.inf
+    h1[162:164] = -np.inf
+    h0[164:166] = np.nan
+    h1[166:168] = np.nan
+    h0[168], h1[168] = -np.inf, 0.0
+    finite = np.r_[0:160, 169:N]
     big = np.float32(1e25)
     grp.projections[0].branches[0].u1.copy_(torch.from_numpy(h0))
     grp.projections[0].branches[1].u1.copy_(torch.from_numpy(h1))
+    rows = np.unique(np.r_[0:40, M - 40:M])  # rows are independent
     for scale in (np.float32(1), big):
         xs = x * float(scale)
-        y = grp.forward(xs)[0].cpu().numpy().astype(np.float64)
-        ref = O.littlebit_forward(xs.cpu().numpy(), [b.as_dict() for b in brs], K, N)
+        y = grp.forward(xs)[0].cpu().numpy().astype(np.float64)[rows]
+        with np.errstate(invalid="ignore"):
+            ref = O.littlebit_forward(xs.cpu().numpy()[rows], [b.as_dict() for b in brs], K, N)
         # per column: each column has its own scale
-        err = np.abs(y - ref).max(0) / np.abs(ref).max(0)
-        print(f"[split] ratios scale={scale:g} worst column {err.max():.2e}", flush=True)
-        assert np.isfinite(y).all() and err.max() <= TOL[torch.float32]
+        err = np.abs(y - ref)[:, finite].max(0) / np.abs(ref[:, finite]).max(0)
+        print(f"[split] M={M} ratios scale={scale:g} worst column {err.max():.2e}", flush=True)
+        assert np.isfinite(y[:, finite]).all() and err.max() <= TOL[torch.float32]
+        assert np.array_equal(y[:, 160:169], ref[:, 160:169], equal_nan=True)
+        assert np.isinf(y[:, 160:164]).all() and np.isnan(y[:, 164:168]).all()
 
 
 @pytest.mark.parametrize("M", [70, 300, 1024])
