@@ -4382,7 +4382,10 @@ static int attn_batch_ch(int heads, int n, int64_t start) {
 //    8 tokens  at 0: 12.6 / 8.8, 1000: 19.2 / 15.1, 1500: 21.3 / 20.0, 2000: 23.3 / 21.4
 //    2 tokens, 8 kv heads  at 40: 12.8 / 9.7, 1000: 13.9 / 13.4, 1300: 14.6 / 19.2, 3500: 18.2 / 32.4
 // so: more than 32 tokens, or many positions (times heads: what the old form's
-// blocks grow with) for groups or more than 16 tokens.  With a device start
+// blocks grow with) for groups or more than 16 tokens (16 without groups
+// lose at 1,000 positions and win 6 % at 1,500, 12 % at 3,000: a line elsewhere,
+// not drawn).
+// Past the 32-bit limits below the old form takes any count up to 64.  With a device start
 // the old form's grid and partials are those of the cache's end, and this one
 // divides the positions there are (25 tokens at 100 of 2,100: 15.1 / 23.0; 8
 // tokens, 8 kv heads: 17.3 / 13.5, of 8,000: 18.5 / 19.5), so the lines are others.
@@ -4429,7 +4432,7 @@ int lbk_attention_batch(const float* q, const float* k, const float* v, float* k
   const size_t need = lbk_attention_batch_partial_bytes(heads, n, sgrid, head_dim);
   if (partial_bytes < need)
     return set_error(LBK_ERR_WORKSPACE, "partial buffer of %zu bytes needed, %zu given", need, partial_bytes);
-  AttnBatchParams p;
+  AttnBatchParams p{};
   p.q = q;
   p.k = k;
   p.v = v;
@@ -4445,10 +4448,6 @@ int lbk_attention_batch(const float* q, const float* k, const float* v, float* k
   p.kvh = kv_heads;
   p.rep = heads / kv_heads;
   p.max_seq = max_seq;
-  p.ch = attn_batch_ch(heads, n, sgrid);
-  p.chunks = int(ceil_div(sgrid + n, p.ch));
-  p.qt = n <= 16 ? 1 : n <= 32 ? 2 : 4;
-  p.ps = 4 / p.qt;
   p.scale = scale;
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (const int chunks = attn_rows_chunks(heads, kv_heads, n, head_dim, sgrid, start_device != nullptr)) {
@@ -4477,6 +4476,10 @@ int lbk_attention_batch(const float* q, const float* k, const float* v, float* k
                                    : (n > 16 ? &attn_rows_kernel<64, 4> : &attn_rows_kernel<64, 8>);
     hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s, r);
   } else {
+    p.ch = attn_batch_ch(heads, n, sgrid);
+    p.chunks = int(ceil_div(sgrid + n, p.ch));
+    p.qt = n <= 16 ? 1 : n <= 32 ? 2 : 4;
+    p.ps = 4 / p.qt;
     const dim3 grid{unsigned(heads), unsigned(p.chunks), 1u};
     if (head_dim == 128) hipLaunchKernelGGL(attn_batch_kernel<128>, grid, dim3(kAttnThreads), 0, s, p);
     else hipLaunchKernelGGL(attn_batch_kernel<64>, grid, dim3(kAttnThreads), 0, s, p);

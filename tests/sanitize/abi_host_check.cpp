@@ -255,6 +255,15 @@ int main() {
     EXPECT(prefill(xf, xf, 65, 32, 8, 128, 1024, 959) == LBK_OK, "prefill up to the cache's end");
     EXPECT(launches.size() == 1 && launches[0].grid.x == (65 * 4 + 31) / 32 * 8, "prefill grid");
   }
+  for (int heads : {65536, 65600}) {  // 2**22 elements per token, and past them
+    launches.clear();
+    EXPECT(lbk_attention_batch(xf, xf, xf, xf, xf, 40, heads, heads, 64, 49, nullptr, 9, nullptr, 1.f, xf,
+                               lbk_attention_batch_partial_bytes(heads, 40, 9, 64), xf, nullptr) == LBK_OK,
+           "batch of %d heads", heads);
+    EXPECT(launches.size() == 2 && launches[0].name.find(heads > 65536 ? "attn_batch_kernel" : "attn_rows_kernel") !=
+                                       std::string::npos,
+           "batch of %d heads runs another kernel", heads);
+  }
   EXPECT(lbk_q4_0_quantize(xf, 4, 33, static_cast<uint8_t*>(ws), static_cast<uint16_t*>(ws), nullptr) == LBK_ERR_ARG,
          "q4 cols % 32");
   EXPECT(lbk_lm_head_q4_workspace_bytes(32000, 4096) > 0, "lm head workspace");

@@ -82,3 +82,32 @@ def test_attention_batch_nothing_seen(gpu):
     assert not out[7].any()
     v[7] = 0
     assert torch.allclose(out, v, rtol=1e-6, atol=0)  # one position each: its own value
+
+
+def test_attention_batch_of_very_many_heads(gpu):
+    """Past 2**22 elements per token the calls of 33 to 64 tokens stay with
+    the kernel that fewer tokens take (the other's offsets are 32-bit): its
+    form of four query tiles, which no smaller shape reaches."""
+    import littlebit_amd._lib as L
+    lib = L.load()
+    n, start, heads, hd = 40, 9, 65600, 64
+    gen = torch.Generator(device=gpu).manual_seed(5)
+    q, k, v = (torch.randn((n, heads * hd), generator=gen, device=gpu) for _ in range(3))
+    kc, vc = (torch.randn((heads, start + n, hd), generator=gen, device=gpu) for _ in range(2))
+    kc[:, start:], vc[:, start:] = float("nan"), float("nan")
+    need = lib.lbk_attention_batch_partial_bytes(heads, n, start, hd)
+    part, out = torch.empty(need // 4, device=gpu), torch.full((n, heads * hd), float("nan"), device=gpu)
+    L.check(lib.lbk_attention_batch(q.data_ptr(), k.data_ptr(), v.data_ptr(), kc.data_ptr(), vc.data_ptr(), n, heads,
+                                    heads, hd, start + n, None, start, None, hd ** -0.5, part.data_ptr(), need,
+                                    out.data_ptr(), torch.cuda.current_stream(gpu).cuda_stream), "lbk_attention_batch")
+    torch.cuda.synchronize()
+    assert torch.equal(kc[:, start:], k.view(n, heads, hd).transpose(0, 1))
+    assert torch.equal(vc[:, start:], v.view(n, heads, hd).transpose(0, 1))
+    sample = torch.randint(0, heads, (64,), generator=gen, device=gpu).tolist() + [0, heads - 1]
+    seen = torch.ones(n, start + n, dtype=torch.bool, device=gpu).tril(start)
+    for h in sample:
+        s = q.view(n, heads, hd)[:, h].double() @ kc[h].double().t().contiguous() * hd ** -0.5
+        ref = torch.softmax(s.masked_fill(~seen, float("-inf")), -1) @ vc[h].double()
+        err = (out.view(n, heads, hd)[:, h] - ref).abs().max().item()
+        assert err <= 2e-5, (h, err)  # (as above)
+    assert not torch.isnan(out).any()
