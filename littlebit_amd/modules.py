@@ -292,10 +292,13 @@ class LittleBitLinear(nn.Linear):
     # forward (littlebit.py:95-121)
     # ------------------------------------------------------------------
     def _projection(self) -> LittleBitProjection:
-        if self._proj is not None:
+        proj = self._proj
+        if proj is not None:
             u = self._buffers.get("U_packed")  # (an attribute lookup on a module costs 1 us)
-            if self._proj.device == (self.U_packed if u is None else u).device:
-                return self._proj
+            if u is None:
+                u = self.U_packed
+            if proj.device == u.device:
+                return proj
         branches = []
         for branch in self._branches():
             sfx = _BRANCH_SUFFIX[branch]
