@@ -176,7 +176,8 @@ class LittleBitDecoder:
             return self._attention_hip(q, k, v, kc, vc, start, pos_t)
         if 1 < N <= 64 and pos_t is None and self._hip_attn and length == start + N:
             return self._attention_batch_hip(q, k, v, kc, vc, start, tree_mask)
-        if N > 64 and tree_mask is None and pos_t is None and self._hip_attn and length == start + N:
+        if (N > 64 and tree_mask is None and pos_t is None and self._hip_attn and length == start + N
+                and not self._prefill_on_library(N, length)):
             return self._attention_prefill_hip(q, k, v, kc, vc, start)
         k3 = k.view(N, kvh, hd).transpose(0, 1)
         v3 = v.view(N, kvh, hd).transpose(0, 1)
@@ -263,6 +264,23 @@ class LittleBitDecoder:
             _raw_stream(q.device.index))
         _lib.check(rc, "lbk_attention_batch")
         return out
+
+    def _prefill_on_library(self, N: int, length: int) -> bool:
+        """Whether a prompt's attention stays with the library's products.
+
+        The kernel has a block per 32 (token, head of the group) rows, which
+        walks all positions (about 35 ns each at head_dim 128, 20 at 64): with
+        few blocks and a long context it leaves the chip idle where a library
+        product splits its sums.  us, kernel / library: 8 heads (2 kv) x 128,
+        65 tokens (18 blocks) after 3,000 positions 117 / 130, 8,000 285 / 142,
+        16,000 560 / 188; 250 tokens (64 blocks) 125 / 146, 291 / 275, 560 / 485;
+        500 tokens (126 blocks) 133 / 234, 300 / 509, 569 / 912.  4 heads (1 kv) x
+        64, 65 tokens (9 blocks) 64 / 131, 158 / 133, 320 / 186.  32 heads (8 kv)
+        x 128, 65 tokens (72 blocks) 119 / 177, 287 / 286, 558 / 561.
+        """
+        c = self.config
+        blocks = c.num_key_value_heads * -(-N * c.kv_repeat // 32)
+        return blocks <= 64 and length > (4096 if c.head_dim == 128 else 6144)
 
     def _attention_prefill_hip(self, q, k, v, kc, vc, start: int):
         """More than 64 new tokens (a prompt), causal, in one launch."""
