@@ -24,12 +24,17 @@
 // product) in 328 us, 1.13 PFLOP/s, where an 8192^3 bf16 library product reaches
 // 1.19 on the same card.  bf16, M = 2048, the Llama-3 gate (4096 -> 14336, ranks
 // 318 + 2867): 240 GFLOP in 240 us, 1.00 PFLOP/s (9 VALU per expanded operand
-// and 2 MFMAs).  A call of few tiles is bound by its chain of steps, about 340
-// cycles each without any memory access (fp32, M = 300, 4096 -> 4096, ranks 205
-// + 1843: 48 us, 0.42 PFLOP/s).  128-row tiles with 64 KB (bf16) or 128 KB
+// and 2 MFMAs).  A call of few tiles is bound by its chain of steps (fp32, M =
+// 300, 4096 -> 4096, ranks 205 + 1843: 48 us, 0.42 PFLOP/s): stage 2's 67 steps
+// take 23 us and stage 1's 43 take 17, about 800 cycles each, of which 340 are
+// the step itself without any memory access; what the rest waits for is not
+// shown (the compiler's wait for all loads in every group of four steps, for the
+// words that two forms of load merge into, is 0.7 us of the 48).  128-row tiles with 64 KB (bf16) or 128 KB
 // (fp32, separate planes, two accumulator sets) of LDS ring, two and one waves
 // per SIMD, took 506, 255 and 94 us for the three, and 43 us against 19 for a
-// bf16 draft projection of rank 205 at M = 300; here a block needs 16 or 32 KB
+// bf16 draft projection of rank 205 at M = 300 (the other way round for bf16 on
+// long rows at many: 14336 -> 4096, ranks 318 + 2867, M = 2048, 832 tiles of 64
+// rows, 289 us against 270 with stream-K); here a block needs 16 or 32 KB
 // of LDS and at most 128 registers, so four waves per SIMD hide each other's LDS
 // reads, barriers and expansions.  A stage of four steps per barrier for the
 // 32-row tiles measured no faster (fp32, M = 300, stage 2: 21.0 -> 23.3 us,
@@ -173,8 +178,8 @@ __global__ __launch_bounds__(kBlock) void sg_scale_kernel(SgParams p) {
 // and group.  A tiles go from global memory straight to LDS through a ring
 // of 4 stages issued 3 steps ahead; 16-byte chunk c of row r is stored at
 // chunk c ^ swz(r), swz(r) = (r ^ (r >> 3)) & 7 (no bank conflicts).  Vector
-// loads complete in issue order, and each step issues the same loads on
-// every path (clamped addresses): W = a group's word loads, F = a fill,
+// loads complete in issue order, and each step of the ring issues the same
+// loads on every path (clamped addresses): W = a group's word loads, F = a fill,
 //   SPLIT: W0 F0 F1 F2 | step 0: W1 F3 | step 1: F4 | step 2: F5 | step 3: F6 | ...
 //   else:  W0 F0 W1 F1 F2 | step 0: W2 F3 | step 1: F4 | step 2: W3 F5 | step 3: F6 | ...
 // so before step ks F(ks) has landed once at most 2 fills and the words
