@@ -2956,7 +2956,12 @@ size_t gemm_ws_bytes(const ProjDesc* pd, int np, int64_t M, int64_t K, int plane
 //   MFMA per product: M = 1024, gate and up, 1536 tiles 72.8 -> 60.1 us; 544
 //   tiles 37.4 us against 41.1 us), and over long rows, in parts for three
 //   blocks per CU (bf16, M = 1024, 11008 -> 4096: 86.2 us against 96.5 us in
-//   768 tiles of 32 rows and 100.1 us in 384 whole tiles of 64).
+//   768 tiles of 32 rows and 100.1 us in 384 whole tiles of 64).  bf16 there in
+//   128-row tiles, two blocks per CU, where 64-row ones would give some CUs a
+//   fourth block for the whole k range (more than 768) and these fit one round
+//   (at most 512): an operand feeds four MFMAs, 14336 -> 4096, ranks 318 + 2867, M
+//   = 2048: 277.7 -> 257.0 us; 2 to 12 % over K = 8192 .. 20480 and 769 .. 1024
+//   tiles of 64; 750 of them 214 us against 226, 1,040 339 against 403.
 //   Stage 2: 32 x 128 tiles while they are few (fp32, M = 512, 4096 columns:
 //   512 tiles 22.2 us, 64 x 128 27.1 us, 64 x 256 43.8 us) or the ranks are
 //   short (each tile then mostly stores y; as long as a launch holds the
@@ -2988,7 +2993,9 @@ SgPlan sg_plan(const ProjDesc* pd, int np, int64_t M, int64_t K, bool split) {
   const int64_t tiles1 = rows1 * c1, tiles2 = (rows1 + 1) / 2 * c1;
   s.mi1 = s.parts = 1;
   int64_t parts = 1;
-  if (K >= 8192 && tiles2 >= 96) {
+  if (!split && K >= 8192 && tiles2 > 768 && ceil_div(M, 128) * c1 <= 512) {
+    s.mi1 = 4;
+  } else if (K >= 8192 && tiles2 >= 96) {
     s.mi1 = 2;
     parts = (768 + tiles2 / 2) / tiles2;
   } else if (tiles1 > (split ? 1500 : 700)) {
@@ -3479,6 +3486,12 @@ void launch_sg_expand(const SgParams& p, const SgPlan& sp, dim3 grid, hipStream_
 }
 template <bool SPLIT, bool GB>
 void launch_sg_latent(const SgParams& p, const SgPlan& sp, dim3 grid, hipStream_t s) {
+  if constexpr (!SPLIT) {
+    if (sp.mi1 == 4) {
+      hipLaunchKernelGGL((sg_latent_kernel<false, GB, 4>), grid, dim3(kBlock), 0, s, p);
+      return;
+    }
+  }
   if (sp.mi1 == 2) hipLaunchKernelGGL((sg_latent_kernel<SPLIT, GB, 2>), grid, dim3(kBlock), 0, s, p);
   else hipLaunchKernelGGL((sg_latent_kernel<SPLIT, GB, 1>), grid, dim3(kBlock), 0, s, p);
 }

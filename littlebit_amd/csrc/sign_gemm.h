@@ -32,11 +32,11 @@
 // words that two forms of load merge into, is 0.7 us of the 48).  128-row tiles with 64 KB (bf16) or 128 KB
 // (fp32, separate planes, two accumulator sets) of LDS ring, two and one waves
 // per SIMD, took 506, 255 and 94 us for the three, and 43 us against 19 for a
-// bf16 draft projection of rank 205 at M = 300 (the other way round for bf16 on
-// long rows at many: 14336 -> 4096, ranks 318 + 2867, M = 2048, 832 tiles of 64
-// rows, 289 us against 270 with stream-K); here a block needs 16 or 32 KB
+// bf16 draft projection of rank 205 at M = 300; here a block needs 16 or 32 KB
 // of LDS and at most 128 registers, so four waves per SIMD hide each other's LDS
-// reads, barriers and expansions.  A stage of four steps per barrier for the
+// reads, barriers and expansions (where stage 1 of a bf16 call has tiles for a
+// little more than three of those blocks per CU over a long K, 128-row tiles of 64
+// KB, two blocks per CU, are the faster ones: figures at sg_plan).  A stage of four steps per barrier for the
 // 32-row tiles measured no faster (fp32, M = 300, stage 2: 21.0 -> 23.3 us,
 // three blocks per CU instead of seven).
 
@@ -392,7 +392,7 @@ __device__ __forceinline__ SgTile sg_tile(const SgParams& p) {
 // -> 3.482e-6 of the result's norm; 1,024 rows 3.502e-6 -> 3.477e-6), no slower
 // (layer of 700 rows 818 -> 810 us).
 template <bool SPLIT, bool GB, int MI>
-__global__ __launch_bounds__(kBlock, 4) void sg_latent_kernel(SgParams p) {
+__global__ __launch_bounds__(kBlock, MI == 4 ? 2 : 4) void sg_latent_kernel(SgParams p) {
   constexpr int NJ = 1;
   constexpr int WPS = SPLIT ? 1 : 2;  // sign words per step
   const int tid = int(threadIdx.x), lane = tid & 63;

@@ -391,6 +391,13 @@ int main() {
         {"64-row tiles, K off", 2049, 264, {{130, 205, 3000}}, F, "Lb1ELb0ELi2E", "IfLb1E", false},
         {"64-row tiles, K off", 2049, 264, {{130, 205, 3000}}, B, "Lb0ELb0ELi2E", "IfLb0E", false},
         {"64-row tiles, odd steps", 2049, 320, {{130, 205, 3000}}, B, "Lb0ELb1ELi2E", "IfLb0E", false},
+        {"128-row tiles", 2049, 8384, {{130, 40, 2900}}, B, "Lb0ELb1ELi4E", "IfLb0E", false},
+        {"128-row tiles, K off", 2049, 8200, {{130, 40, 2900}}, B, "Lb0ELb0ELi4E", "IfLb0E", false},
+        {"bf16 long rows", 2048, 14336, {{4096, 318, 2867}}, B, "Lb0ELb1ELi4E", "IfLb0E", false},
+        {"bf16 long rows, 768 tiles", 2048, 11008, {{4096, 298, 2686}}, B, "Lb0ELb1ELi2E", "IfLb0E", false},
+        {"bf16 long rows, 520 tiles of 128", 2500, 11008, {{4096, 318, 2867}}, B, "Lb0ELb1ELi2E", "IfLb0E", false},
+        {"fp32 long rows", 2048, 14336, {{4096, 318, 2867}}, F, "Lb1ELb0ELi2E", "IfLb1E", false},
+        {"bf16 shorter rows", 2048, 4096, {{4096, 318, 2867}}, B, "Lb0ELb1ELi2E", "IfLb0E", false},
         {"64 x 128", 1100, 200, {{5000, 40, 600}}, F, "Lb1E", "IfLb1ELi2ELi1E", false},
         {"64 x 256", 1100, 200, {{9000, 40, 601}}, F, "Lb1E", "IfLb1ELi2ELi2E", false},
         {"32 x 128", 200, 260, {{4500, 40, 600}}, F, "Lb1E", "IfLb1ELi1ELi1E", false},

@@ -16,7 +16,7 @@ import pytest
 from littlebit_amd.build import LIB_PATH
 
 OBJDUMP = Path(os.environ.get("ROCM_PATH", "/opt/rocm")) / "llvm" / "bin" / "llvm-objdump"
-KERNELS = [f"sg_latent_kernelILb{s}ELb{g}ELi{mi}E" for s, g in ((1, 0), (0, 1), (0, 0)) for mi in (1, 2)] + [
+KERNELS = [f"sg_latent_kernelILb{s}ELb{g}ELi{mi}E" for s, g in ((1, 0), (0, 1), (0, 0)) for mi in (1, 2, 4)[:3 - s]] + [
     f"sg_expand_kernelI{y}Lb{s}ELi{mi}ELi{nj}E" for y in "ft" for s in (0, 1) for mi, nj in ((1, 1), (2, 1), (2, 2))]
 
 

@@ -55,6 +55,8 @@ def _check(host, specs, K, x, outs, rows=None, tol=TOL[torch.float32]):
     (2049, 264, [(130, [205, 3000])]),              # stage 1 as 64-row tiles
     (2049, 320, [(130, [205, 3000])]),              # the same, bf16 rows read as they are, an odd step
     (330, 8256, [(130, [205, 1843])]),              # long rows: 64-row tiles in parts
+    (2049, 8384, [(130, [40, 2900])]),              # long rows, bf16 as 128-row tiles: three steps past the ring's rounds
+    (2049, 8200, [(130, [40, 2900])]),              # the same from a scaled copy (K off the steps)
 ])
 def test_sign_gemm_edges(gpu, M, K, specs, x_dtype):
     """(Which kernels these shapes run is checked in tests/sanitize/abi_host_check.cpp.)"""
